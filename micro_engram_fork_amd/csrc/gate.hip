@@ -38,7 +38,9 @@
 // DPP row shifts and combines the two column waves in LDS. Workgroup ids are remapped so the
 // 32 CUs of one XCD work on a compact group of tiles (8 token tiles x 4 column tiles) and share
 // their operands in that XCD's L2. bf16 forward passes run the same scheme on 256 x 224 tiles
-// of 16x16x32 MFMAs (gate224_kernel: whole rounds of tiles on the Gemma-scale shape).
+// of 16x16x32 MFMAs (gate224_kernel: whole rounds of tiles on the Gemma-scale shape), and so does
+// the plain projection of me_kv_proj (kProj: the K loop with K or V rows stored in its epilogue;
+// 8192 tokens x 5376 x 1536, both weights: 233 us, 1.16 PFLOP/s).
 #include "me_common.h"
 
 #include <mutex>
@@ -68,13 +70,17 @@ constexpr uint32_t kBufferConfig = 0x00020000u;    // raw buffer descriptor word
 constexpr int kStoreNT = 2;                        // buffer store cache policy bit: non-temporal
 static_assert(4 * kWaveStage + 2 * kTile * 3 * 4 <= kRingBytes, "epilogue must fit in the ring");
 
-// Forward passes (key, value) and the backward's two passes over the same GEMM tiles.
-enum Phase : int { kKey = 0, kValue = 1, kGradValue = 2, kGradKey = 3 };
+// Forward passes (key, value), the backward's two passes over the same GEMM tiles, and the plain
+// projection (K and V rows written out, gate224_kernel only).
+enum Phase : int { kKey = 0, kValue = 1, kGradValue = 2, kGradKey = 3, kProj = 4 };
 
 struct GateArgs {
     const uint8_t *hidden;  // [n, d] of H
     const uint8_t *mem;     // [n, m] of T
     const uint8_t *w;       // [d, m] of T (W_K in the key pass, W_V in the value pass)
+    const uint8_t *w2;      // projection: [d, m] W_V (w is W_K)
+    uint8_t *kv;            // projection: [n, 2d] of T, K | V
+    uint32_t kv_bytes;
     const void *q_delta;    // [d] scale - 1 (nullable: scalar gate)
     const void *k_delta;
     const uint8_t *keep;    // [n] (nullable)
@@ -740,13 +746,15 @@ __global__ __launch_bounds__(kThreads, 1) void gate224_kernel(const GateArgs a) 
     const int first_nt = group * kGroupTiles;
     const int group_nts = min(kGroupTiles, a.n_nt - first_nt);
     const int nt = first_nt + in_group % group_nts;
-    const int jt = in_group / group_nts;
+    const int jt_all = in_group / group_nts;  // projection: W_K's column tiles, then W_V's
+    const bool second = PHASE == kProj && 2 * jt_all >= a.n_jt;
+    const int jt = second ? jt_all - a.n_jt / 2 : jt_all;
+    const uint8_t *w = second ? a.w2 : a.w;
     const int64_t j0 = static_cast<int64_t>(jt) * kTJ;
     const int64_t n0 = static_cast<int64_t>(nt) * kTile;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wj = wave >> 1, wn = wave & 1;
-
 
     // ---- epilogue row walk geometry: 14 of 16 lanes x 16 bytes per token row (the wave's 112
     // columns), lane l16 owning 8 columns, rows rsub, rsub + 4, ... of the wave's 128 tokens
@@ -841,7 +849,7 @@ __global__ __launch_bounds__(kThreads, 1) void gate224_kernel(const GateArgs a) 
     // ---- K loop over 128-byte slabs: A_s (W rows) in unit 2s % 5, B_s (mem rows) in (2s+1) % 5
     const uint32_t row_bytes = static_cast<uint32_t>(a.m * sizeof(T));
     const int slabs = static_cast<int>(ceil_div(row_bytes, kSlab));
-    const int32x4 rsrc_w = buffer_rsrc(a.w, a.w_bytes);
+    const int32x4 rsrc_w = buffer_rsrc(w, a.w_bytes);
     const int32x4 rsrc_m = buffer_rsrc(a.mem, a.mem_bytes);
     // A load i of a wave fills rows 8 (7 wave + i) + [0, 8), B load i rows 8 (8 wave + i) + [0, 8):
     // lane l writes row + l / 8 at physical chunk l % 8 (logical chunk (l % 8) ^ ((row >> 1) & 7)).
@@ -1020,7 +1028,7 @@ __global__ __launch_bounds__(kThreads, 1) void gate224_kernel(const GateArgs a) 
 #pragma unroll
         for (int u = 0; u < 32; ++u)
             xpre[u] = __builtin_bit_cast(u32x4_v, __builtin_amdgcn_raw_buffer_load_b128(rg, row_off(u), 0, 0));
-    } else {
+    } else if constexpr (PHASE == kGradKey) {
         if (a.q_delta != nullptr) load_scales();
     }
     if (parts_late && n_tok < a.n) {
@@ -1044,7 +1052,7 @@ __global__ __launch_bounds__(kThreads, 1) void gate224_kernel(const GateArgs a) 
         s_aux[tid] = alpha_reg;
     } else if (PHASE == kKey) {
         for (int e = tid; e < 2 * kTile * 3; e += kThreads) s_aux[e] = 0.f;
-    } else {
+    } else if (PHASE == kGradKey) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) s_aux[tid * 3 + c] = coef_reg[c];
     }
@@ -1097,7 +1105,23 @@ __global__ __launch_bounds__(kThreads, 1) void gate224_kernel(const GateArgs a) 
             cw[0] = c0.x; cw[1] = c0.y; cw[2] = c1.x; cw[3] = c1.y;
         }
     };
-    if constexpr (PHASE != kGradKey) {
+    if constexpr (PHASE == kProj) {
+        // 16 bytes per lane and row into the K or V half of the token's K | V row; a row past n or a
+        // lane past d stores nothing (its offset is the range end)
+        const __amdgpu_buffer_rsrc_t rkv =
+            __builtin_amdgcn_make_buffer_rsrc(a.kv, 0, static_cast<int>(a.kv_bytes), kBufferConfig);
+        const uint32_t o0 =
+            jok ? static_cast<uint32_t>(((ntok0 + rsub) * 2 * a.d + (second ? a.d : 0) + jl) * 2) : 0u;
+        const uint32_t ostride = static_cast<uint32_t>(a.d * 16);  // four rows
+#pragma unroll
+        for (int u = 0; u < 32; ++u) {
+            uint32_t cw[4];
+            staged(u * 4 + rsub, cw);
+            __builtin_amdgcn_raw_buffer_store_b128(
+                u32x4_v{cw[0], cw[1], cw[2], cw[3]}, rkv,
+                4 * u < rows_left ? o0 + static_cast<uint32_t>(u) * ostride : a.kv_bytes, 0, 0);
+        }
+    } else if constexpr (PHASE != kGradKey) {
 #pragma unroll
         for (int u = 0; u < 32; ++u) {
             const int row = u * 4 + rsub;
@@ -1402,6 +1426,30 @@ int gate_common(GateArgs &a, const void *hidden, int hidden_dtype, int64_t n, in
 }  // namespace me
 
 using namespace me;
+
+// K | V rows of me_kv_proj on the fused gate's 256 x 224 tiles (proj.hip picks between these and its
+// own): bf16, whole 128-byte slabs of the memory rows, at least three of them.
+int me::kv_proj_224(const void *mem, int64_t n, int64_t mem_dim, const void *w_key, const void *w_value,
+                    int64_t model_dim, void *kv, hipStream_t s) {
+    GateArgs a{};
+    a.mem = static_cast<const uint8_t *>(mem);
+    a.w = static_cast<const uint8_t *>(w_key);
+    a.w2 = static_cast<const uint8_t *>(w_value);
+    a.kv = static_cast<uint8_t *>(kv);
+    a.kv_bytes = static_cast<uint32_t>(n * model_dim * 4);
+    a.n = n;
+    a.d = model_dim;
+    a.m = mem_dim;
+    a.mem_bytes = static_cast<uint32_t>(n * mem_dim * 2);
+    a.w_bytes = static_cast<uint32_t>(model_dim * mem_dim * 2);
+    a.n_jt = 2 * static_cast<int>(ceil_div(model_dim, kTJ));
+    a.n_nt = static_cast<int>(ceil_div(n, kTile));
+    a.total_tiles = a.n_jt * a.n_nt;
+    a.per_xcd = static_cast<int>(ceil_div(a.total_tiles, kXcds));
+    hipLaunchKernelGGL(gate224_kernel<kProj>, dim3(static_cast<unsigned>(a.per_xcd * kXcds)), dim3(kThreads),
+                       0, s, a);
+    return check_launch("me_kv_proj (256 x 224 tiles)");
+}
 
 extern "C" int me_gate_workspace_size(int64_t n, int64_t model_dim, size_t *bytes) {
     ME_CHECK_ARG(bytes != nullptr, "bytes is null");

@@ -120,6 +120,10 @@ __device__ __forceinline__ gmem_ptr<T> as_global_addr(uint64_t addr) {
 
 // ---------------------------------------------------------------------------------------------
 // Launch helpers.
+// me_kv_proj on the gate's 256 x 224 tiles (gate.hip): checked arguments, bf16.
+int kv_proj_224(const void *mem, int64_t n, int64_t mem_dim, const void *w_key, const void *w_value,
+                int64_t model_dim, void *kv, hipStream_t s);
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -1,12 +1,12 @@
-// Stage 3 for few tokens on gfx950: the key and value projections of the memory vectors,
+// Stage 3 on gfx950: the key and value projections of the memory vectors,
 //   kv[n][j]     = round_T(sum_m mem[n][m] W_K[j][m])        j < d
 //   kv[n][d + j] = round_T(sum_m mem[n][m] W_V[j][m])        j < d
-// the two nn.Linear calls of MicroEngram.inject (micro_engram/module.py:245, 254), for batches
-// too small for the fused gate kernel's 256 x 224 tiles to fill the part (a serving decode step:
-// 256 tokens against 10,752 output columns of K = 1536). me_gate_rows then does the gate and
-// the residual add from kv.
+// the two nn.Linear calls of MicroEngram.inject (micro_engram/module.py:245, 254). me_gate_rows
+// then does the gate and the residual add from kv. Batches that fill the part with the fused gate
+// kernel's 256 x 224 tiles take those (gate.hip); the tiles here are for smaller ones (a serving
+// decode step: 256 tokens against 10,752 output columns of K = 1536).
 //
-// At this size the GEMM is bound by moving operands into the CUs: the weights (33 MB at the
+// At that size the GEMM is bound by moving operands into the CUs: the weights (33 MB at the
 // Gemma-scale shape) are read once per token tile, the memory vectors once per column tile.
 // Measured on MI355X, loads that ask each 128-byte line for half of it (what an MFMA fragment
 // loaded straight into registers is: 16 rows x 64 bytes) move the same bytes 1.5x slower than
@@ -295,21 +295,37 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     a.mem_bytes = static_cast<uint32_t>(n * mem_dim * es);
     a.w_bytes = static_cast<uint32_t>(model_dim * mem_dim * es);
     hipStream_t s = as_stream(stream);
-    // Tiles (measured on MI355X at model dim 5376, mem dim 1536, bf16): small batches are
-    // bound by how many bytes each CU keeps in flight from L2, so they take tiles whose ring
-    // leaves room for two workgroups per CU (four slots of 128-byte slabs) -- up to 64 tokens
+    // Tiles (measured on MI355X at model dim 5376, mem dim 1536, bf16, unless said otherwise): small
+    // batches are bound by how many bytes each CU keeps in flight from L2, so they take tiles whose
+    // ring leaves room for two workgroups per CU (four slots of 128-byte slabs) -- up to 64 tokens
     // 32 x 96 (10.8 us against 12.8 us with one 64 x 96 workgroup per CU), up to 256 tokens
     // 64 x 96 (a 256-token decode step's projection: 15.8-16.0 us against 17.8 us with 128 x 96
-    // and a five-slot ring; 128 x 64, 64 x 128 and 32 x 96 there: 17-20 us) -- and larger batches
-    // the 128 x 192 tile, which moves the fewest bytes per MFMA (512 tokens 26.8 us, 1024 tokens
-    // 50 us). fp32 (model dim 1024, mem dim 1024): small tiles fill the CUs and two workgroups
+    // and a five-slot ring; 128 x 64, 64 x 128 and 32 x 96 there: 17-20 us). Larger batches take
+    // the gate's 256 x 224 tiles (one workgroup per CU, a matrix core's worth of work per barrier)
+    // or 64 x 128 ones (three slots, two workgroups per CU), whichever needs the less time for the
+    // whole rounds its tiles make on 256 CUs: a round of the first takes about 7 us and 1.25 us per
+    // slab, 256 tiles of the second 1.2 us and 0.33 us per slab, but never under 1.6 such (512
+    // tokens: 33.4 and 30.5 us; 768: 33.7, 36.7; 1237: 39.0, 61.6; 2048: 69.9, 101; 8192: 233, 398;
+    // at 2048 x 1024, 1024 tokens: 24.8, 14.9; 2048: 25.7, 27.1; 8192: 76.7, 107; at 1024 x 512, 2048
+    // tokens: 16.9, 10.6). Both were measured against 128 x 192 tiles (512 tokens 29.2 us, 1024: 51.5,
+    // 1237: 73.2, 8192: 363), which stay for many tokens of a memory width the first cannot take.
+    // fp32 (model dim 1024, mem dim 1024): small tiles fill the CUs and two workgroups
     // share one -- up to 768 tokens 32 x 64 (256 tokens 16.7 us against 72.5 with 128 x 128),
     // up to 1024 32 x 128 (40.9 us), above 64 x 128 with a three-slot ring (2048 tokens 72.3 us
     // against 74.8, 8192 tokens 276 against 295).
     if (dtype == ME_BF16) {
         if (n <= 64) return launch<uint16_t, 1, 3, 4>(a, s);
         if (n <= 256) return launch<uint16_t, 2, 3, 4>(a, s);
-        return launch<uint16_t, 4, 6, 4>(a, s);
+        constexpr int64_t kCus = 256;
+        const float small = static_cast<float>(ceil_div(ceil_div(n, 64) * ceil_div(2 * a.d_pad, 128), kCus));
+        if (a.row_bytes % kSlab == 0 && a.slabs >= 3 && n * model_dim * 4 < (int64_t{1} << 31)) {
+            const float large = static_cast<float>(ceil_div(ceil_div(n, 256) * 2 * ceil_div(model_dim, 224), kCus));
+            if (large * (7.f + 1.25f * a.slabs) <= 2.f + fmaxf(small, 1.6f) * (1.2f + 0.33f * a.slabs))
+                return kv_proj_224(mem, n, mem_dim, w_key, w_value, model_dim, kv, s);
+        } else if (ceil_div(n, 128) * ceil_div(2 * a.d_pad, 192) > 2 * kCus) {
+            return launch<uint16_t, 4, 6, 4>(a, s);
+        }
+        return launch<uint16_t, 2, 4, 3>(a, s);
     }
     if (n <= 768) return launch<float, 1, 2, 5>(a, s);
     if (n <= 1024) return launch<float, 1, 4, 4>(a, s);

@@ -14,9 +14,9 @@ Differences from the reference, all deliberate:
   * lookup() returns views into one concatenated [N, n_tables * D] buffer instead of separate
     tensors per table (same values).
   * Where a gradient is needed (grad mode on and hidden or a parameter requiring it), the
-    forward keeps the memory vectors and per-token gate sums, and the backward runs the HIP
-    gate backward (the projections recomputed on MFMA) plus four plain GEMMs for the weight and
-    memory gradients; the table gradients go through the dedup kernel (rows.py). Without
+    forward keeps the memory vectors, K and V (up to keep_kv_bytes) and per-token gate sums, and
+    the backward runs the HIP gate backward (the projections recomputed on MFMA where they were
+    not kept) and the kernels of the weight and memory gradients; the table gradients go through the dedup kernel (rows.py). Without
     gradients, hashing and the gather run fused and nothing is kept.
   * The "ple" gate keeps its parameters (so checkpoints load) but has no HIP kernel.
 """
@@ -96,32 +96,48 @@ class _GateResidual(torch.autograd.Function):
     """hidden + the gated projection of the memory vectors (module.py:239-261) with its
     gradients: the HIP backward gives the gradients of hidden, of the key / value Linear
     outputs and of the scale deltas; the Linear layers' own gradients (dW = dY^T mem,
-    dmem = dY_K W_K + dY_V W_V) come from _linear_grads."""
+    dmem = dY_K W_K + dY_V W_V) come from _linear_grads.
+
+    keep_kv: K and V are written out by the projection kernel and kept for the backward, as autograd
+    keeps the two nn.Linear outputs, and the gate and its backward are one pass over the rows each;
+    else (K and V too large to keep) the fused kernels compute them tile by tile, again in the
+    backward."""
 
     @staticmethod
-    def forward(ctx, hidden, mem, w_key, w_value, q_delta, k_delta, gate_mode, keep):
-        out, alpha, stats = ops.gate_residual(
-            hidden, mem, w_key.detach(), w_value.detach(),
-            None if q_delta is None else q_delta.detach(),
-            None if k_delta is None else k_delta.detach(), gate_mode, keep, True, True)
-        ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats)
+    def forward(ctx, hidden, mem, w_key, w_value, q_delta, k_delta, gate_mode, keep, keep_kv):
+        q = None if q_delta is None else q_delta.detach()
+        k = None if k_delta is None else k_delta.detach()
+        kv = None
+        if keep_kv:
+            d = hidden.shape[-1]
+            kv = ops.kv_proj(mem, w_key.detach(), w_value.detach())
+            out, alpha, stats = ops.gate_rows(hidden, kv[:, :d], kv[:, d:], q, k, gate_mode, keep, True, True)
+        else:
+            out, alpha, stats = ops.gate_residual(hidden, mem, w_key.detach(), w_value.detach(), q, k,
+                                                  gate_mode, keep, True, True)
+        ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv)
         ctx.gate_mode = gate_mode
         ctx.mark_non_differentiable(alpha)
         return out, alpha
 
     @staticmethod
     def backward(ctx, grad_out, _grad_alpha):
-        hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats = ctx.saved_tensors
+        hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv = ctx.saved_tensors
         need = ctx.needs_input_grad
         wk, wv = w_key.detach(), w_value.detach()
-        g_hidden, g_key, g_value, g_q, g_k = ops.gate_backward(
-            grad_out.contiguous(), hidden.detach(), mem.detach(), wk, wv,
-            None if q_delta is None else q_delta.detach(),
-            None if k_delta is None else k_delta.detach(), ctx.gate_mode, keep, stats)
+        q = None if q_delta is None else q_delta.detach()
+        k = None if k_delta is None else k_delta.detach()
+        if kv is not None:
+            d = hidden.shape[-1]
+            g_hidden, g_key, g_value, g_q, g_k = ops.gate_rows_backward(
+                grad_out.contiguous(), hidden.detach(), kv[:, :d], kv[:, d:], q, k, ctx.gate_mode, keep, stats)
+        else:
+            g_hidden, g_key, g_value, g_q, g_k = ops.gate_backward(
+                grad_out.contiguous(), hidden.detach(), mem.detach(), wk, wv, q, k, ctx.gate_mode, keep, stats)
         d_mem, d_wk, d_wv = _linear_grads(g_key, g_value, mem.detach(), wk, wv, need[1:4])
         d_q = g_q.to(q_delta.dtype) if need[4] else None
         d_k = g_k.to(k_delta.dtype) if need[5] else None
-        return g_hidden if need[0] else None, d_mem, d_wk, d_wv, d_q, d_k, None, None
+        return g_hidden if need[0] else None, d_mem, d_wk, d_wv, d_q, d_k, None, None, None
 
 
 def _linear_grads(g_key, g_value, mem, wk, wv, need):
@@ -461,10 +477,12 @@ class MicroEngram(nn.Module):
         mode = ME_GATE_SCALAR_SQRT if sqrt else ME_GATE_SCALAR
         fits = ops.fits_mfma(hidden.shape[-1], mem.shape[-1], mem.dtype)
         if self._needs_grad(hidden) or mem.requires_grad:
-            fn = _GateResidual if fits else _GateResidualRows
-            out, alpha = fn.apply(hidden, mem, self.key.weight, self.value.weight,
-                                  self.q_scale if sqrt else None, self.k_scale if sqrt else None,
-                                  mode, keep)
+            args = (hidden, mem, self.key.weight, self.value.weight,
+                    self.q_scale if sqrt else None, self.k_scale if sqrt else None, mode, keep)
+            if fits:
+                out, alpha = _GateResidual.apply(*args, self._keeps_kv(hidden, mem))
+            else:
+                out, alpha = _GateResidualRows.apply(*args)
             if self.training:
                 self._record_gate(alpha)
             return out
@@ -483,7 +501,8 @@ class MicroEngram(nn.Module):
             limit = self.few_tokens_max
         else:  # also bounded by the fp32 K|V rows the few-token path writes ([N, 2d])
             limit = min(self.few_tokens_max_fp32, self.few_tokens_kv_bytes // (8 * hidden.shape[-1]))
-        if n_tok <= limit:
+        if n_tok <= limit or (limit > 0 and mem.dtype == hidden.dtype == torch.bfloat16
+                              and ops.prefers_rows(n_tok, hidden.shape[-1], mem.shape[-1])):
             outs = ops.gate_residual_rows(hidden, mem, self.key.weight.detach(), self.value.weight.detach(),
                                           q, k, mode, keep, self.training)
         else:
@@ -493,11 +512,13 @@ class MicroEngram(nn.Module):
             self._record_gate(outs[1])
         return outs[0]
 
-    # Token counts up to which the gate without gradients runs the key and value projections
-    # in the few-token kernel (me_kv_proj) and the gate in the row kernel (me_gate_rows) instead
-    # of the fused kernel, whose 256-token tiles come in whole rounds of the CUs and leave many
-    # of them idle below the last round. Measured on MI355X (model dim 5376, memory dim 1536,
-    # bf16): 256 tokens 33 us against 73, 1024 tokens 61 against 74, 1536 tokens 88 against 76.
+    # Token counts up to which the gate without gradients always runs the key and value projections
+    # in a kernel of their own (me_kv_proj) and the gate in the row kernel (me_gate_rows) instead of
+    # the fused kernel, whose 256-token tiles come in whole rounds of the CUs and leave many of
+    # them idle below the last round; 0 keeps every call on the fused kernels. Measured on MI355X
+    # (model dim 5376, memory dim 1536, bf16): 256 tokens 25 us against 73, 1025 tokens 48 against
+    # 77. Above, bf16 calls take the faster of the two by the rounds their tiles make
+    # (ops.prefers_rows).
     # fp32 engrams: the fused kernel's fp32 tiles are 256 x 256 on 32x32x2 MFMAs, so a 2048-token
     # batch (model dim 1024) gives it 32 tiles per pass (538 us) and the few-token path (72 us for
     # the projection) stays ahead far longer. That range was measured at model dim 1024 only, so
@@ -506,6 +527,19 @@ class MicroEngram(nn.Module):
     few_tokens_max = 1024
     few_tokens_max_fp32 = 16384
     few_tokens_kv_bytes = 128 << 20
+
+    # Bytes of K and V (the key / value Linear outputs, [N, 2d]) up to which a forward with
+    # gradients keeps them for the backward. That saves the backward's two recomputing passes: a
+    # training step of 8192 tokens at model dim 5376 (bf16, 176 MB) takes 1.20 ms against 1.44,
+    # forward and backward of 2048 fp32 tokens at 1024 0.92 against 1.43.
+    keep_kv_bytes = 1 << 30
+
+    def _keeps_kv(self, hidden, mem):
+        """Whether a forward with gradients writes K and V out and keeps them (few_tokens_max = 0 keeps
+        every call on the fused kernels, with or without gradients)."""
+        few = self.few_tokens_max if mem.dtype == torch.bfloat16 else self.few_tokens_max_fp32
+        n = hidden.numel() // hidden.shape[-1]
+        return n < 1 << 24 and few > 0 and 2 * hidden.numel() * mem.element_size() <= self.keep_kv_bytes
 
     def inject(self, hidden, idx, keep=None):
         """hidden + gated memory of the rows `idx` (module.py:228-261); keep: optional [N] bool,

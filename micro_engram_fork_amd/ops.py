@@ -432,12 +432,37 @@ def fits_mfma(model_dim, mem_dim, dtype):
     return model_dim % 8 == 0 and (mem_dim * esize) % 16 == 0
 
 
+def prefers_rows(n, model_dim, mem_dim):
+    """Whether the gate of n bf16 tokens without gradients is faster as projection (kv_proj) + row
+    kernel (gate_rows) than in the fused kernel, for shapes both take (whole 128-byte slabs of the
+    memory rows, at least three).
+
+    Both run 256 x 224 tiles, one per CU, so their time goes by whole rounds of 256 tiles: the fused
+    kernel makes one set of rounds per pass (key, value), the projection one set for both together,
+    then K and V cross the memory once each way. A round of the fused kernel's two passes takes
+    about 25 us and 2.2 us per slab, one of the projection 7 and 1.25 (or less on small tiles),
+    the row kernel 8 bytes per token and column at 5.3 TB/s. Measured at model dim 5376, memory dim
+    1536, fused / rows: 1237 tokens 75 / 50 us, 2048: 81 / 86, 4096: 164 / 155, 8192: 268 / 293; at
+    2048 x 1024, 2048: 59 / 36, 4096: 62 / 72, 8192: 119 / 106; at 1024 x 512, 4096: 43 / 30."""
+    slabs = mem_dim * 2 // 128
+    if mem_dim * 2 % 128 or slabs < 3 or n * model_dim * 4 >= 1 << 31:
+        return False
+    tiles = -(-n // 256) * -(-model_dim // 224)
+    small = -(-(-(-n // 64) * -(-model_dim // 64)) // 256)
+    proj = min(-(-2 * tiles // 256) * (7 + 1.25 * slabs), 2 + max(small, 1.6) * (1.2 + 0.33 * slabs))
+    return proj + 2.5 + n * model_dim * 8 / 5.3e6 < -(-tiles // 256) * (25 + 2.2 * slabs)
+
+
 def _kv_rows(k, v, d):
-    """K and V rows for the row kernels: one stride for both (contiguous [N, d] tensors)."""
-    k, v = k.reshape(-1, d).contiguous(), v.reshape(-1, d).contiguous()
+    """(K rows, V rows, their row stride in elements) for the row kernels: [N, d] tensors as they are
+    when their rows are contiguous and one stride apart (the halves of kv_proj's [N, 2d]), else
+    contiguous copies."""
     if k.dtype != v.dtype:
         raise ValueError("[micro_engram] K and V rows must share one dtype")
-    return k, v
+    k, v = k.reshape(-1, d), v.reshape(-1, d)
+    if k.stride(1) == v.stride(1) == 1 and k.stride(0) == v.stride(0) >= d:
+        return k, v, k.stride(0)
+    return k.contiguous(), v.contiguous(), d
 
 
 @_custom_op("gate_rows")
@@ -451,7 +476,7 @@ def gate_rows(hidden: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     d = hidden.shape[-1]
     x = hidden.reshape(-1, d).contiguous()
     N = x.shape[0]
-    k, v = _kv_rows(k, v, d)
+    k, v, kv_stride = _kv_rows(k, v, d)
     if k.shape[0] != N:
         raise ValueError(f"[micro_engram] K/V rows {tuple(k.shape)} do not match {N} tokens")
     q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode)
@@ -459,7 +484,7 @@ def gate_rows(hidden: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     out = torch.empty_like(x)
     alpha = torch.empty(N, dtype=torch.float32, device=dev) if with_alpha else None
     stats = torch.empty((N, 4), dtype=torch.float32, device=dev) if with_stats else None
-    call("me_gate_rows", x.data_ptr(), dtype_code(x), N, d, k.data_ptr(), v.data_ptr(), d,
+    call("me_gate_rows", x.data_ptr(), dtype_code(x), N, d, k.data_ptr(), v.data_ptr(), kv_stride,
          dtype_code(k), _p(q_scale_delta), _p(k_scale_delta), scale_code, gate_mode, _p(keep_u8),
          out.data_ptr(), _p(alpha), _p(stats), stream_of(dev))
     res = [out.reshape(hidden.shape)]
@@ -493,7 +518,7 @@ def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Te
     d = hidden.shape[-1]
     x = hidden.reshape(-1, d).contiguous()
     N = x.shape[0]
-    k, v = _kv_rows(k, v, d)
+    k, v, kv_stride = _kv_rows(k, v, d)
     g = grad_out.reshape(-1, d).to(x.dtype).contiguous()
     stats = stats.contiguous()
     if tuple(stats.shape) != (N, 4) or stats.dtype != torch.float32:
@@ -509,7 +534,7 @@ def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Te
     size = ctypes.c_size_t(0)
     call("me_gate_rows_backward_workspace_size", N, d, ctypes.byref(size))
     ws = torch.empty(max(size.value, 16), dtype=torch.uint8, device=dev)
-    call("me_gate_rows_backward", x.data_ptr(), dtype_code(x), N, d, k.data_ptr(), v.data_ptr(), d,
+    call("me_gate_rows_backward", x.data_ptr(), dtype_code(x), N, d, k.data_ptr(), v.data_ptr(), kv_stride,
          dtype_code(k), _p(q_scale_delta), _p(k_scale_delta), scale_code, gate_mode, _p(keep_u8),
          g.data_ptr(), stats.data_ptr(), grad_hidden.data_ptr(), grad_k.data_ptr(),
          grad_v.data_ptr(), grad_q.data_ptr() if sqrt else None, grad_kd.data_ptr() if sqrt else None,

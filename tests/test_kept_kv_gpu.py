@@ -1,0 +1,96 @@
+"""The projection + row kernels that a forward with gradients runs (K and V written out and kept)
+against the fused kernels: the same K and V bits, the same sums in the same order, so every output
+but the scale gradients (sums over tokens in another order) is equal bit for bit.
+
+Scale gradients: both are fp32 sums of the same n terms t_i = a_i x_i K_i, each within
+n * 2^-24 * sum |t_i| of the exact one (a few ulps more for the products), so their difference is
+held to twice that; sum |t_i| is bounded by sqrt(n) times the columns' 2-norm, and the terms here
+are random in sign: |difference| <= 1e-5 * 2-norm over columns covers n = 2049 with a wide margin
+against observed 2e-7."""
+import pytest
+import torch
+
+from micro_engram_fork_amd import MicroEngram, ops
+from micro_engram_fork_amd._lib import ME_GATE_SCALAR, ME_GATE_SCALAR_SQRT
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _case(n, d, m, mode, dtype, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g, device=DEV) * std).to(dtype)
+    scales = (r(d, std=0.1), r(d, std=0.1)) if mode == ME_GATE_SCALAR_SQRT else (None, None)
+    return (r(n, d), r(n, m, std=0.05), r(d, m, std=0.05), r(d, m, std=0.05), *scales,
+            torch.rand(n, generator=g, device=DEV) > 0.1, r(n, d, std=1e-3))
+
+
+# model dims: one group of 8 columns, one column past a 224-column tile, an odd number of 112-column
+# halves, every step count of the row kernels (up to 24, 48 and 72 groups of 112), past them (8072)
+@pytest.mark.parametrize("n,d,m,mode", [
+    (1, 8, 192, ME_GATE_SCALAR_SQRT), (3, 112, 192, ME_GATE_SCALAR), (257, 232, 192, ME_GATE_SCALAR_SQRT),
+    (513, 1032, 512, ME_GATE_SCALAR_SQRT), (2049, 336, 256, ME_GATE_SCALAR_SQRT),
+    (255, 2688, 256, ME_GATE_SCALAR_SQRT), (256, 2696, 256, ME_GATE_SCALAR), (300, 5376, 1536, ME_GATE_SCALAR_SQRT),
+    (5, 5384, 192, ME_GATE_SCALAR_SQRT), (70, 8064, 192, ME_GATE_SCALAR_SQRT), (70, 8072, 192, ME_GATE_SCALAR_SQRT)])
+def test_rows_equal_fused_bf16(n, d, m, mode):
+    x, mem, wk, wv, dq, dk, keep, g = _case(n, d, m, mode, torch.bfloat16)
+    fused = ops.gate_residual(x, mem, wk, wv, dq, dk, mode, keep, True, True)
+    kv = ops.kv_proj(mem, wk, wv)
+    rows = ops.gate_rows(x, kv[:, :d], kv[:, d:], dq, dk, mode, keep, True, True)
+    if d <= 8064:
+        for a, b in zip(fused, rows):
+            assert torch.equal(a, b)
+    stats = fused[2]
+    want = ops.gate_backward(g, x, mem, wk, wv, dq, dk, mode, keep, stats)
+    got = ops.gate_rows_backward(g, x, kv[:, :d], kv[:, d:], dq, dk, mode, keep, stats)
+    if d <= 8064:
+        for a, b in zip(want[:3], got[:3]):
+            assert torch.equal(a, b)
+    for a, b in zip(want[3:], got[3:]):
+        assert (a - b).norm() <= 1e-5 * a.norm() + 1e-12
+
+
+# token counts around the switches between the projection's tiles (64, 256 tokens; then by the
+# rounds they make: 64 x 128 or 256 x 224 tiles) and memory widths of whole and partial slabs
+@pytest.mark.parametrize("n", [64, 65, 256, 257, 512, 513, 768, 1025])
+@pytest.mark.parametrize("d,m", [(5376, 192), (264, 1536), (2048, 200)])
+def test_kv_proj_tiles(n, d, m):
+    _, mem, wk, wv, *_ = _case(n, d, m, ME_GATE_SCALAR, torch.bfloat16, seed=n)
+    kv = ops.kv_proj(mem, wk, wv)
+    ref = torch.cat([mem.double() @ wk.double().t(), mem.double() @ wv.double().t()], dim=1)
+    mag = torch.cat([mem.double().abs() @ wk.double().abs().t(), mem.double().abs() @ wv.double().abs().t()], dim=1)
+    # one rounding to bf16 of an fp32 sum of m exact products
+    assert bool(((kv.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + m * 2.0 ** -24 * mag).all())
+
+
+def _make(dtype, d, tables=6, dim=32):
+    torch.manual_seed(d)
+    eng = MicroEngram(model_dim=d, table_size=257, engram_dim=dim, num_heads=tables // 2, orders=(2, 3),
+                      vocab_size=1000, gate="scalar_sqrt")
+    torch.nn.init.normal_(eng.value.weight, std=0.1)
+    return eng.to(device=DEV, dtype=dtype).train()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("hidden_dtype", [torch.bfloat16, torch.float32])
+def test_kept_and_recomputed_gradients_agree(dtype, hidden_dtype):
+    # above keep_kv_bytes the backward recomputes K and V; both give the same gradients
+    n, d = 300, 264
+    eng = _make(dtype, d)
+    ids = torch.randint(0, 1000, (1, n), device=DEV)
+    g = torch.randn(1, n, d, device=DEV).to(hidden_dtype) * 1e-2
+    hidden = torch.randn(1, n, d, device=DEV).to(hidden_dtype)
+    grads = []
+    for limit in (1 << 30, 0):
+        eng.keep_kv_bytes = limit
+        eng.zero_grad(set_to_none=True)
+        h = hidden.clone().requires_grad_(True)
+        out = eng(h, ids)
+        assert (out.grad_fn is not None)
+        out.backward(g)
+        grads.append([out.detach(), h.grad] + [p.grad for p in eng.parameters()])
+    # bf16: K, V, dK and dV round the same values, differing by their sums' order; near s = 0 the
+    # square root's slope carries that into a token's gradients, hence 5e-2 of the 2-norm there
+    tol = 5e-2 if torch.bfloat16 in (dtype, hidden_dtype) else 5e-3
+    for a, b in zip(*grads):
+        assert a.dtype == b.dtype and (a.double() - b.double()).norm() <= tol * b.double().norm() + 1e-12
