@@ -353,6 +353,23 @@ int me_dedup_table_bounds(const int64_t *uniq, int64_t n, const int64_t *count,
                           int64_t *info, void *stream);
 
 /*
+ * me_dense_table_grads -- the dense gradients of plain embedding tables from a row lookup's
+ * coalesced ones: grads[k][r] = the sum of unique row r of table k, rounded to dtype, or zero for a
+ * row no lookup touched (what the autograd of nn.Embedding leaves for module.py:146-154), all
+ * tables in one launch.
+ *
+ *   local_rows, info   as me_dedup_table_bounds or me_dedup_tables leave them (rows ascending and
+ *                      unique per table, each in [0, table_rows[k]))
+ *   sums       fp32 [count, dim]: the summed gradient row of each unique row (me_dedup_sums);
+ *              both may be NULL when info counts no rows
+ *   grads      HOST array of n_tables device pointers, [table_rows[k], dim] of dtype (ME_BF16 /
+ *              ME_F32), every element written; NULL: no gradient wanted for that table
+ */
+int me_dense_table_grads(const int64_t *local_rows, const float *sums, const int64_t *info,
+                         int32_t n_tables, const int64_t *table_rows, int32_t dim, int dtype,
+                         void *const *grads, void *stream);
+
+/*
  * me_dedup_tables -- the key half of a row lookup's dedup from its per-table row ids, and the
  * tables' bounds in it: what me_dedup_keys + me_dedup_table_bounds give for the token-major keys
  * offset_k + idx[k][t] (lookup position t * n_tables + k), in two launches for up to 8,192

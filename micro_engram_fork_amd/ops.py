@@ -803,6 +803,19 @@ def dedup_table_bounds(uniq, count, offsets):
     return local, info
 
 
+def dense_table_grads(local_rows, sums, info, shapes, dtype, need):
+    """The dense gradient of every table k with need[k] (None for the others), [rows_k, D] of dtype:
+    its unique rows' sums in their places, zero elsewhere (the nn.Embedding gradients of
+    module.py:146-154), all tables in one launch. local_rows and info as dedup_tables or
+    dedup_table_bounds give them, sums as dedup_sums; no count is read on the host."""
+    dev = require_gpu(local_rows, sums, info)
+    grads = [torch.empty(shape, dtype=dtype, device=dev) if n else None for shape, n in zip(shapes, need)]
+    call("me_dense_table_grads", _p(local_rows), _p(sums), info.data_ptr(), len(shapes),
+         i64_array([int(shape[0]) for shape in shapes]), shapes[0][1], _DTYPES[dtype],
+         ptr_array([_p(g) for g in grads]), stream_of(dev))
+    return grads
+
+
 def dedup_tables(idx2d, table_rows, inverse=True):
     """[uniq, local rows, inv, count, plan, info] of the token-major lookups of per-table row ids
     idx2d [n_tables, n] (key offset_k + idx2d[k, t] at position t * n_tables + k): what

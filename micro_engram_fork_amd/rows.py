@@ -104,29 +104,34 @@ class _KeyPlan:
     asynchronous copy with an event behind it, so the backward's host read waits for the plan
     only, not for the gate's backward and the weight products queued before it."""
 
-    def __init__(self, idx2d, offsets):
-        self.idx2d, self.offsets, self.outs = idx2d, offsets, None
+    def __init__(self, idx2d, offsets, to_host=True):
+        self.idx2d, self.offsets, self.outs, self.host = idx2d, offsets, None, None
+        self.to_host = to_host  # the bounds are wanted on the host (sparse gradients)
 
     def make(self):
         if self.outs is None:
             rows = [b - a for a, b in zip(self.offsets, self.offsets[1:])]
             uniq, self.local_all, inv, count, plan, info = ops.dedup_tables(self.idx2d, rows, inverse=False)
             self.outs = [uniq, inv, count, plan]  # inv unwritten: the segment sums read the plan
-            self.host = _pinned_take(info.numel())
-            self.host.copy_(info, non_blocking=True)
-            self.ready = torch.cuda.Event()
-            self.ready.record(torch.cuda.current_stream(info.device))  # the copy's stream
+            self.info = info
+            if self.to_host:
+                self.host = _pinned_take(info.numel())
+                self.host.copy_(info, non_blocking=True)
+                self.ready = torch.cuda.Event()
+                self.ready.record(torch.cuda.current_stream(info.device))  # the copy's stream
             self.idx2d = None
         return self.outs
 
     def bounds(self):
-        """(local rows of the unique keys, [count, table bounds] as host ints)."""
+        """[count, table bounds] as host ints."""
         self.make()
+        if self.host is None:
+            return self.info.tolist()
         self.ready.synchronize()
         buf, self.host = self.host, None
         host = buf.tolist()
         _pinned_give(buf)  # its copy is done and read (a plan that is never read keeps its own)
-        return self.local_all, host
+        return host
 
 
 _PINNED = {}
@@ -185,7 +190,7 @@ class _RowLookup(torch.autograd.Function):
         ctx.shards = shards if any(getattr(s, "_sparse_rows", False) for s in shards) else None
         ctx.plan = None
         if any(ctx.needs_input_grad[2:]) and idx2d.numel() > 0:
-            ctx.plan = _KeyPlan(idx2d, offsets)
+            ctx.plan = _KeyPlan(idx2d, offsets, ctx.shards is not None)
             pending = getattr(_PLANS, "pending", None)
             if pending is None:
                 ctx.plan.make()
@@ -200,29 +205,36 @@ class _RowLookup(torch.autograd.Function):
         D = ctx.shapes[0][0][1]
         offs_all = _offsets_on(ctx.offsets, idx2d.device)
         offs = offs_all[:-1]
-        if ctx.plan is not None:  # the key half and the bounds ran in the forward
-            uniq_all, inv, count, plan = ctx.plan.make()
-            outs = [uniq_all, inv, count, ops.dedup_sums(plan, count, grad.reshape(n * nt, D))]
-            local_all, host = ctx.plan.bounds()
-            ctx.plan = None
+        need = ctx.needs_input_grad[2:]
+        sparse = [n and ctx.shards is not None and getattr(ctx.shards[k], "_sparse_rows", False)
+                  for k, n in enumerate(need)]
+        dense = [n and not s for n, s in zip(need, sparse)]
+        plan = ctx.plan
+        if plan is not None:  # the key half and the bounds ran in the forward
+            _uniq, _inv, count, keys = plan.make()
+            gsum = ops.dedup_sums(keys, count, grad.reshape(n * nt, D))
+            local_all, info = plan.local_all, plan.info
         else:
-            outs = ops.dedup(_lookup_keys(idx2d, offs), int(ctx.offsets[-1]), grad.reshape(n * nt, D))
+            _uniq, _inv, count, gsum = ops.dedup(_lookup_keys(idx2d, offs), int(ctx.offsets[-1]),
+                                                 grad.reshape(n * nt, D))
+            local_all, info = ops.dedup_table_bounds(_uniq, count, ctx.offsets)
+        if any(dense):  # device side throughout: no count is read on the host
+            dtype = ctx.shapes[0][1]
+            grads = ops.dense_table_grads(local_all, gsum, info, [s for s, _ in ctx.shapes], dtype, dense)
+        else:
+            grads = [None] * nt
+        if any(sparse):
             # one host read for the unique count and every table's bounds
-            local_all, info = ops.dedup_table_bounds(outs[0], outs[2], ctx.offsets)
-            host = info.tolist()
-        cnt, bounds = host[0], host[1:]
-        # each table's slice of the unique rows and sums (bounds[0] = 0, bounds[nt] = count)
-        sizes = [bounds[k + 1] - bounds[k] for k in range(nt)]
-        locals_ = local_all[:cnt].split(sizes)
-        sums = outs[3][:cnt].split(sizes)
-        batch = SparseBatch(local_all[:cnt], outs[3][:cnt], bounds)
-        grads = []
-        for k, (shape, dtype) in enumerate(ctx.shapes):
-            if not ctx.needs_input_grad[2 + k]:
-                grads.append(None)
-                continue
-            if ctx.shards is not None and getattr(ctx.shards[k], "_sparse_rows", False):
-                shard = ctx.shards[k]
+            host = plan.bounds() if plan is not None else info.tolist()
+            cnt, bounds = host[0], host[1:]
+            # each table's slice of the unique rows and sums (bounds[0] = 0, bounds[nt] = count)
+            sizes = [bounds[k + 1] - bounds[k] for k in range(nt)]
+            locals_ = local_all[:cnt].split(sizes)
+            sums = gsum[:cnt].split(sizes)
+            batch = SparseBatch(local_all[:cnt], gsum[:cnt], bounds)
+            for k, shard in enumerate(ctx.shards):
+                if not sparse[k]:
+                    continue
                 if getattr(shard, "sparse_grad", None) is None:
                     # this table's part of the dedup is already coalesced: unique rows in
                     # ascending order and fp32 sums that start from +0.0, as index_add_'s do
@@ -230,11 +242,7 @@ class _RowLookup(torch.autograd.Function):
                     shard.sparse_grad = batch.member(shard, k, locals_[k], sums[k])
                 else:
                     add_sparse_grad(shard, locals_[k], sums[k])
-                grads.append(None)
-                continue
-            g = torch.zeros(shape, dtype=torch.float32, device=grad.device)
-            g[locals_[k]] = sums[k]  # unique rows: a plain scatter
-            grads.append(g.to(dtype))
+        ctx.plan = None
         return (None, None, *grads)
 
 
