@@ -249,6 +249,133 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     }
 }
 
+// ---- a few tokens: every weight byte in flight at once ---------------------------------------------
+// Up to kFewTokens tokens the GEMM is one read of the weights (33 MB at the Gemma-scale shape) and next to
+// no arithmetic, so what counts is how soon all of it is in flight: a tile's ring (above) keeps three
+// slabs of its rows in flight and walks 24, a chain of eight memory latencies. Here a workgroup takes
+// 16 columns whole: its four waves split the slabs, each wave asks for all of its rows' lines at
+// once (buffer_load ... lds, whole lines) and for its token fragments (into registers; a few KB
+// that every workgroup reads, so L2 has them), waits once, multiplies, and the waves' partial tiles
+// are added in wave order. At 24 slabs a workgroup holds 48 KB of LDS, so three share a CU and the
+// 672 workgroups of the Gemma-scale shape are all resident. One token there: 7.3 us, 4.5 TB/s of weights
+// with the launch in it (10.2 us in 32 x 96 ring tiles); at 2048 x 1024 3.8 us (7.6), at 1024 x 1024 in
+// fp32 4.7 (16.0).
+// SW: slabs per wave at most; B: 16-token blocks.
+template <typename T, int SW, int B>
+__global__ __launch_bounds__(kThreads) void proj_few_kernel(const ProjArgs a) {
+    constexpr int kEs = sizeof(T);
+    constexpr int kOwn = SW * 2048;  // bytes of a wave's rows
+    __shared__ __attribute__((aligned(16))) uint8_t lds[4 * kOwn];
+    static_assert(4 * kOwn <= kLdsBytes, "rows fit LDS");
+    static_assert(kOwn >= B * 1024, "a wave's partial tiles fit where its rows were");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t vc0 = static_cast<int64_t>(blockIdx.x) * 16;  // virtual column: K block, then V block
+    const bool is_v = vc0 >= a.d_pad;
+    const int64_t j0 = is_v ? vc0 - a.d_pad : vc0;
+    const int32x4 rw = rsrc_of(is_v ? a.wv : a.wk, a.w_bytes);
+    const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(a.mem), 0, static_cast<int>(a.mem_bytes), kBufferConfig);
+    const int sw = (a.slabs + 3) / 4;
+    const int s0 = wave * sw, ns = min(sw, a.slabs - s0);  // this wave's slabs (none if ns <= 0)
+    // token fragments: lane l holds token 16 b + (l & 15), chunk 4 ks + (l >> 4) of a slab
+    const int fr = lane & 15, fq = lane >> 4;
+    u32x4_v fa[B][SW][2];
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int i = 0; i < SW; ++i)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const int64_t t = 16 * b + fr;
+                const uint32_t kb = static_cast<uint32_t>(s0 + i) * kSlab + static_cast<uint32_t>(4 * ks + fq) * 16u;
+                const uint32_t off = t < a.n && i < ns && kb < a.row_bytes ? static_cast<uint32_t>(t) * a.row_bytes + kb
+                                                                          : a.mem_bytes;
+                fa[b][i][ks] = __builtin_bit_cast(u32x4_v, __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0));
+            }
+    __builtin_amdgcn_sched_barrier(0);
+    uint8_t *own = lds + wave * kOwn;
+    const uint32_t own_lds = lds_addr(own);
+#pragma unroll
+    for (int i = 0; i < 2 * SW; ++i) {  // 8 rows of a slab: lane l takes row 8 (i & 1) + l / 8, chunk swizzled
+        if (i / 2 < ns) {
+            const int row = 8 * (i & 1) + (lane >> 3);
+            const uint32_t kb = static_cast<uint32_t>(s0 + i / 2) * kSlab +
+                                static_cast<uint32_t>((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+            const uint32_t off = j0 + row < a.d && kb < a.row_bytes
+                                     ? static_cast<uint32_t>(j0 + row) * a.row_bytes + kb
+                                     : a.w_bytes;
+            dma16(rw, __builtin_amdgcn_readfirstlane(own_lds + static_cast<uint32_t>(i) * 1024u), off);
+        }
+    }
+    floatx4 acc[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+    wait_vmcnt<0>();  // the wave's own rows and fragments; no other wave reads them
+#pragma unroll
+    for (int i = 0; i < SW; ++i)
+        if (i < ns)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const int c = ((4 * ks + fq) ^ ((fr >> 1) & 7)) << 4;
+                const u32x4_v fb = *reinterpret_cast<const u32x4_v *>(own + i * 2048 + fr * kSlab + c);
+#pragma unroll
+                for (int b = 0; b < B; ++b) Mma<T>::run(acc[b], fa[b][i][ks], fb);
+            }
+    // partial tiles [16 B tokens][16 columns] where the wave's rows were (its reads are done: the
+    // MFMAs above used them)
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            reinterpret_cast<float *>(own)[(16 * b + 4 * fq + r) * 16 + fr] = acc[b][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < B * 128; e += kThreads) {  // two columns of a token
+        const int tok = e >> 3, col = (e & 7) * 2;
+        if (tok >= a.n || j0 + col >= a.d) continue;
+        float v0 = 0.f, v1 = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float *p = reinterpret_cast<const float *>(lds + w * kOwn) + tok * 16 + col;
+            v0 += p[0];
+            v1 += p[1];
+        }
+        uint8_t *o = a.kv + (tok * 2 * a.d + (is_v ? a.d : 0) + j0 + col) * kEs;
+        if constexpr (kEs == 2)
+            *as_global(reinterpret_cast<uint32_t *>(o)) =
+                static_cast<uint32_t>(float_to_bf16_bits_rne(v0)) |
+                (static_cast<uint32_t>(float_to_bf16_bits_rne(v1)) << 16);
+        else
+            *as_global(reinterpret_cast<u32x2_v *>(o)) = u32x2_v{__float_as_uint(v0), __float_as_uint(v1)};
+    }
+}
+
+template <typename T, int B>
+int launch_few(const ProjArgs &a, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(2 * a.d_pad / 16));
+    const int sw = (a.slabs + 3) / 4;
+    if (sw <= 2) hipLaunchKernelGGL((proj_few_kernel<T, 2, B>), grid, dim3(kThreads), 0, s, a);
+    else if (sw <= 4) hipLaunchKernelGGL((proj_few_kernel<T, 4, B>), grid, dim3(kThreads), 0, s, a);
+    else if (sw <= 6) hipLaunchKernelGGL((proj_few_kernel<T, 6, B>), grid, dim3(kThreads), 0, s, a);
+    else if (sw <= 8) hipLaunchKernelGGL((proj_few_kernel<T, 8, B>), grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL((proj_few_kernel<T, 12, B>), grid, dim3(kThreads), 0, s, a);
+    return check_launch("me_kv_proj (few tokens)");
+}
+
+// Every workgroup reads every token's row, so the kernel pays while those reads are few: it takes 64
+// tokens of at most kFewBytes in all (us, few / ring tiles of 32 x 32; model dim x memory dim, bf16:
+// 5376 x 1536, 8 tokens 7.9 / 9.2, 16: 9.2 / 9.2, 32: 13.6 / 9.2; 2048 x 1024, 32: 5.2 / 6.1, 48: 6.8 / 6.2)
+// and rows of at most 48 slabs (96 KB of LDS).
+constexpr int64_t kFewTokens = 64;
+constexpr int64_t kFewBytes = 22'000'000;
+
+template <typename T>
+int few(const ProjArgs &a, hipStream_t s) {
+    if (a.n <= 16) return launch_few<T, 1>(a, s);
+    if (a.n <= 32) return launch_few<T, 2>(a, s);
+    return launch_few<T, 4>(a, s);
+}
+
 template <typename T, int BA, int BB, int R>
 int launch(ProjArgs a, hipStream_t s) {
     constexpr int TM = 32 * BA, TN = 32 * BB;
@@ -296,12 +423,12 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     a.w_bytes = static_cast<uint32_t>(model_dim * mem_dim * es);
     hipStream_t s = as_stream(stream);
     // Tiles (measured on MI355X at model dim 5376, mem dim 1536, bf16, unless said otherwise): small
-    // batches are bound by how many bytes each CU keeps in flight from L2, so they take tiles whose
-    // ring leaves room for two workgroups per CU (four slots of 128-byte slabs) -- up to 64 tokens
-    // 32 x 96 (10.8 us against 12.8 us with one 64 x 96 workgroup per CU), up to 256 tokens
-    // 64 x 96 (a 256-token decode step's projection: 15.8-16.0 us against 17.8 us with 128 x 96
-    // and a five-slot ring; 128 x 64, 64 x 128 and 32 x 96 there: 17-20 us). Larger batches take
-    // the gate's 256 x 224 tiles (one workgroup per CU, a matrix core's worth of work per barrier)
+    // batches are bound by how many bytes each CU keeps in flight from L2, so they take the
+    // smallest tile whose tiles all find a place at once, two workgroups per CU: 32 x 32 with six slots of
+    // 128-byte slabs (19 tokens: 9.2 us; 10.4 with 32 x 96 and four slots; at 2048 x 1024, 128
+    // tokens: 6.9, 8.9), 64 x 64 with four (192 tokens: 13.2; 15.6 with 64 x 96; at 3584 x 1536, 256
+    // tokens: 12.7, 15.4), 64 x 96 with four (256 tokens: 16.0; 64 x 64 20.3, 128 x 96 17.6). Larger
+    // batches take the gate's 256 x 224 tiles (one workgroup per CU, a matrix core's worth of work per barrier)
     // or 64 x 128 ones (three slots, two workgroups per CU), whichever needs the less time for the
     // whole rounds its tiles make on 256 CUs: a round of the first takes about 7 us and 1.25 us per
     // slab, 256 tiles of the second 1.2 us and 0.33 us per slab, but never under 1.6 such (512
@@ -313,16 +440,20 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // share one -- up to 768 tokens 32 x 64 (256 tokens 16.7 us against 72.5 with 128 x 128),
     // up to 1024 32 x 128 (40.9 us), above 64 x 128 with a three-slot ring (2048 tokens 72.3 us
     // against 74.8, 8192 tokens 276 against 295).
+    if (n <= kFewTokens && a.slabs <= 48 && 2 * a.d_pad / 16 * n * a.row_bytes <= kFewBytes)
+        return dtype == ME_BF16 ? few<uint16_t>(a, s) : few<float>(a, s);
     if (dtype == ME_BF16) {
-        if (n <= 64) return launch<uint16_t, 1, 3, 4>(a, s);
-        if (n <= 256) return launch<uint16_t, 2, 3, 4>(a, s);
         constexpr int64_t kCus = 256;
-        const float small = static_cast<float>(ceil_div(ceil_div(n, 64) * ceil_div(2 * a.d_pad, 128), kCus));
+        auto tiles = [&](int tokens, int cols) { return ceil_div(n, tokens) * ceil_div(2 * a.d_pad, cols); };
+        if (tiles(32, 32) <= 2 * kCus) return launch<uint16_t, 1, 1, 6>(a, s);
+        if (tiles(64, 64) <= 2 * kCus) return launch<uint16_t, 2, 2, 4>(a, s);
+        if (tiles(64, 96) <= 2 * kCus) return launch<uint16_t, 2, 3, 4>(a, s);
+        const float small = static_cast<float>(ceil_div(tiles(64, 128), kCus));
         if (a.row_bytes % kSlab == 0 && a.slabs >= 3 && n * model_dim * 4 < (int64_t{1} << 31)) {
             const float large = static_cast<float>(ceil_div(ceil_div(n, 256) * 2 * ceil_div(model_dim, 224), kCus));
             if (large * (7.f + 1.25f * a.slabs) <= 2.f + fmaxf(small, 1.6f) * (1.2f + 0.33f * a.slabs))
                 return kv_proj_224(mem, n, mem_dim, w_key, w_value, model_dim, kv, s);
-        } else if (ceil_div(n, 128) * ceil_div(2 * a.d_pad, 192) > 2 * kCus) {
+        } else if (tiles(128, 192) > 2 * kCus) {
             return launch<uint16_t, 4, 6, 4>(a, s);
         }
         return launch<uint16_t, 2, 4, 3>(a, s);

@@ -349,12 +349,7 @@ def _gate_operands(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, ga
         if not (_aligned(q_scale_delta) and _aligned(k_scale_delta)):
             q_scale_delta, k_scale_delta = q_scale_delta.clone(), k_scale_delta.clone()
         scale_code = dtype_code(q_scale_delta)
-    keep_u8 = None
-    if keep is not None:
-        keep_u8 = keep.reshape(-1).to(torch.uint8).contiguous()
-        if keep_u8.numel() != N:
-            raise ValueError(f"[micro_engram] keep has {keep_u8.numel()} entries for {N} tokens")
-    return x, mem, w_key, w_value, q_scale_delta, k_scale_delta, scale_code, keep_u8, N, d, M
+    return x, mem, w_key, w_value, q_scale_delta, k_scale_delta, scale_code, _keep_u8(keep, N), N, d, M
 
 
 @_custom_op("gate_residual")
@@ -565,7 +560,8 @@ def _scales(q_scale_delta, k_scale_delta, gate_mode):
 def _keep_u8(keep, n):
     if keep is None:
         return None
-    keep_u8 = keep.reshape(-1).to(torch.uint8).contiguous()
+    keep = keep.reshape(-1)  # a bool's byte is what the kernels test: no copy
+    keep_u8 = (keep.view(torch.uint8) if keep.dtype == torch.bool else keep.to(torch.uint8)).contiguous()
     if keep_u8.numel() != n:
         raise ValueError(f"[micro_engram] keep has {keep_u8.numel()} entries for {n} tokens")
     return keep_u8

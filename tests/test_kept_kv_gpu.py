@@ -26,12 +26,13 @@ def _case(n, d, m, mode, dtype, seed=0):
 
 
 # model dims: one group of 8 columns, one column past a 224-column tile, an odd number of 112-column
-# halves, every step count of the row kernels (up to 24, 48 and 72 groups of 112), past them (8072)
+# halves, every step count of the row kernels (up to 24, 48 and 72 groups of 112), past them (8072);
+# more than 64 tokens, where the projection sums over k in the fused kernel's order
 @pytest.mark.parametrize("n,d,m,mode", [
-    (1, 8, 192, ME_GATE_SCALAR_SQRT), (3, 112, 192, ME_GATE_SCALAR), (257, 232, 192, ME_GATE_SCALAR_SQRT),
+    (65, 8, 192, ME_GATE_SCALAR_SQRT), (66, 112, 192, ME_GATE_SCALAR), (257, 232, 192, ME_GATE_SCALAR_SQRT),
     (513, 1032, 512, ME_GATE_SCALAR_SQRT), (2049, 336, 256, ME_GATE_SCALAR_SQRT),
     (255, 2688, 256, ME_GATE_SCALAR_SQRT), (256, 2696, 256, ME_GATE_SCALAR), (300, 5376, 1536, ME_GATE_SCALAR_SQRT),
-    (5, 5384, 192, ME_GATE_SCALAR_SQRT), (70, 8064, 192, ME_GATE_SCALAR_SQRT), (70, 8072, 192, ME_GATE_SCALAR_SQRT)])
+    (69, 5384, 192, ME_GATE_SCALAR_SQRT), (70, 8064, 192, ME_GATE_SCALAR_SQRT), (70, 8072, 192, ME_GATE_SCALAR_SQRT)])
 def test_rows_equal_fused_bf16(n, d, m, mode):
     x, mem, wk, wv, dq, dk, keep, g = _case(n, d, m, mode, torch.bfloat16)
     fused = ops.gate_residual(x, mem, wk, wv, dq, dk, mode, keep, True, True)
@@ -50,17 +51,32 @@ def test_rows_equal_fused_bf16(n, d, m, mode):
         assert (a - b).norm() <= 1e-5 * a.norm() + 1e-12
 
 
-# token counts around the switches between the projection's tiles (64, 256 tokens; then by the
-# rounds they make: 64 x 128 or 256 x 224 tiles) and memory widths of whole and partial slabs
-@pytest.mark.parametrize("n", [64, 65, 256, 257, 512, 513, 768, 1025])
-@pytest.mark.parametrize("d,m", [(5376, 192), (264, 1536), (2048, 200)])
-def test_kv_proj_tiles(n, d, m):
-    _, mem, wk, wv, *_ = _case(n, d, m, ME_GATE_SCALAR, torch.bfloat16, seed=n)
+def _check_proj(n, d, m, dtype):
+    _, mem, wk, wv, *_ = _case(n, d, m, ME_GATE_SCALAR, dtype, seed=n)
     kv = ops.kv_proj(mem, wk, wv)
     ref = torch.cat([mem.double() @ wk.double().t(), mem.double() @ wv.double().t()], dim=1)
     mag = torch.cat([mem.double().abs() @ wk.double().abs().t(), mem.double().abs() @ wv.double().abs().t()], dim=1)
-    # one rounding to bf16 of an fp32 sum of m exact products
-    assert bool(((kv.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + m * 2.0 ** -24 * mag).all())
+    # an fp32 sum of m products (each rounded once more in fp32), then one rounding to bf16
+    rounding = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    assert bool(((kv.double() - ref).abs() <= rounding * ref.abs() + (m + 1) * 2.0 ** -24 * mag).all())
+
+
+# token counts around the switches between the projection's tiles (by the tiles they make: 32 x 32,
+# 64 x 64, 64 x 96, then 64 x 128 or 256 x 224) and memory widths of whole and partial slabs
+@pytest.mark.parametrize("n", [64, 65, 192, 193, 256, 257, 512, 513, 768, 1025])
+@pytest.mark.parametrize("d,m", [(5376, 192), (264, 1536), (2048, 200)])
+def test_kv_proj_tiles(n, d, m):
+    _check_proj(n, d, m, torch.bfloat16)
+
+
+# the few-token kernel: every count of 16-token blocks and its edges, columns that end inside a
+# 16-column block, memory rows of one part of a slab, of fewer slabs than waves, of partial slabs,
+# of each slab count per wave (2, 4, 6, 8, 12) and past its widest (3200)
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("d,m", [(8, 16), (24, 192), (1032, 200), (40, 896), (264, 1536), (16, 2048), (8, 3072), (8, 3200)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_kv_proj_few_tokens(n, d, m, dtype):
+    _check_proj(n, d, m, dtype)
 
 
 def _make(dtype, d, tables=6, dim=32):
