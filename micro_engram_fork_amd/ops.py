@@ -51,7 +51,7 @@ def stream_of(device):
     return torch._C._cuda_getCurrentRawStream(index)
 
 
-_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_PLAIN_TENSORS = frozenset((torch.Tensor, torch.nn.Parameter))
 
 
 def _plain(value):
@@ -74,8 +74,8 @@ def _direct_call(args, kwargs):
         if tp in _PLAIN_TENSORS or a is None:
             continue
         if tp is list or tp is tuple:
-            for v in a:
-                if isinstance(v, torch.Tensor) and type(v) not in _PLAIN_TENSORS:
+            for tp in set(map(type, a)) - _PLAIN_TENSORS:  # one pass in C over 24 tables
+                if issubclass(tp, torch.Tensor):
                     return False
         elif isinstance(a, torch.Tensor):
             return False
@@ -313,6 +313,7 @@ def _(ids, canon, mults, table_orders, table_rows, pad_id, tables, with_idx, ide
 
 
 # ----------------------------------------------------------------------------- gate + residual
+@functools.lru_cache(maxsize=64)
 def gate_workspace_bytes(n, d):
     size = ctypes.c_size_t(0)
     call("me_gate_workspace_size", n, d, ctypes.byref(size))
@@ -501,6 +502,13 @@ def _(hidden, k, v, q_scale_delta, k_scale_delta, gate_mode, keep, with_alpha, w
     return res
 
 
+@functools.lru_cache(maxsize=64)
+def gate_rows_backward_workspace_bytes(n, d):
+    size = ctypes.c_size_t(0)
+    call("me_gate_rows_backward_workspace_size", n, d, ctypes.byref(size))
+    return size.value
+
+
 @_custom_op("gate_rows_backward")
 def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Tensor,
                        v: torch.Tensor, q_scale_delta: Optional[torch.Tensor],
@@ -526,9 +534,7 @@ def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Te
     sqrt = gate_mode == _lib.ME_GATE_SCALAR_SQRT
     grad_q = torch.empty(d if sqrt else 0, dtype=torch.float32, device=dev)
     grad_kd = torch.empty(d if sqrt else 0, dtype=torch.float32, device=dev)
-    size = ctypes.c_size_t(0)
-    call("me_gate_rows_backward_workspace_size", N, d, ctypes.byref(size))
-    ws = torch.empty(max(size.value, 16), dtype=torch.uint8, device=dev)
+    ws = torch.empty(max(gate_rows_backward_workspace_bytes(N, d), 16), dtype=torch.uint8, device=dev)
     call("me_gate_rows_backward", x.data_ptr(), dtype_code(x), N, d, k.data_ptr(), v.data_ptr(), kv_stride,
          dtype_code(k), _p(q_scale_delta), _p(k_scale_delta), scale_code, gate_mode, _p(keep_u8),
          g.data_ptr(), stats.data_ptr(), grad_hidden.data_ptr(), grad_k.data_ptr(),
@@ -610,6 +616,7 @@ def _(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, gate_mode, keep
     return res
 
 
+@functools.lru_cache(maxsize=64)
 def gate_backward_workspace_bytes(n, d):
     size = ctypes.c_size_t(0)
     call("me_gate_backward_workspace_size", n, d, ctypes.byref(size))
@@ -812,6 +819,15 @@ def dense_table_grads(local_rows, sums, info, shapes, dtype, need):
     return grads
 
 
+@functools.lru_cache(maxsize=64)
+def _dedup_tables_args(n, table_rows):
+    """(row counts, workspace bytes) of me_dedup_tables for n lookups in each of these tables."""
+    rows = i64_array(list(table_rows))
+    size = ctypes.c_size_t(0)
+    call("me_dedup_tables_workspace_size", n, len(table_rows), rows, ctypes.byref(size))
+    return rows, size.value
+
+
 def dedup_tables(idx2d, table_rows, inverse=True):
     """[uniq, local rows, inv, count, plan, info] of the token-major lookups of per-table row ids
     idx2d [n_tables, n] (key offset_k + idx2d[k, t] at position t * n_tables + k): what
@@ -824,13 +840,11 @@ def dedup_tables(idx2d, table_rows, inverse=True):
         idx2d = idx2d.long().contiguous()
     nt, n = idx2d.shape
     N = n * nt
-    rows = i64_array([int(r) for r in table_rows])
+    rows, ws_bytes = _dedup_tables_args(n, tuple(int(r) for r in table_rows))
     ints = torch.empty(3 * N + nt + 2, dtype=torch.int64, device=dev)  # four outputs, one allocation
     uniq, local, inv, info = ints[:N], ints[N:2 * N], ints[2 * N:3 * N], ints[3 * N:]
     plan = torch.empty(max(dedup_plan_bytes(N), 16), dtype=torch.uint8, device=dev)
-    size = ctypes.c_size_t(0)
-    call("me_dedup_tables_workspace_size", n, nt, rows, ctypes.byref(size))
-    ws = torch.empty(max(size.value, 16), dtype=torch.uint8, device=dev)
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     call("me_dedup_tables", idx2d.data_ptr() if N else None, idx2d.stride(0) if n else 0, n, nt, rows,
          _p(uniq) if N else None, _p(local) if N else None, _p(inv) if N and inverse else None, info.data_ptr(),
          plan.data_ptr(), plan.numel(), ws.data_ptr(), ws.numel(), stream_of(dev))
