@@ -12,6 +12,7 @@ import contextlib
 import os
 import threading
 
+import numpy as np
 import torch
 
 from . import ops
@@ -291,19 +292,21 @@ class RowTables:
         ps = [p for p in self.params() if p.requires_grad]
         if not ps:
             return None
-        sq = torch.zeros(1, dtype=torch.float32, device=ps[0].device)
         batch, ks = SparseBatch.common(ps) if all(p.grad is None for p in ps) else (None, None)
         if (batch is not None and sorted(ks) == list(range(len(batch.bounds) - 1))
                 and batch.sums.is_contiguous() and batch.sums.data_ptr() % 16 == 0):
             # every table's gradient is its slice of one backward's sums, which tile them
             span = batch.sums.reshape(-1)
-            ops.sumsq(span, sq, accumulate=True)
+            sq = torch.empty(1, dtype=torch.float32, device=span.device)
+            ops.sumsq(span, sq)
             if max_norm and max_norm > 0:
                 ops.clip_scale(span, sq, max_norm)
             if self.optimizer is not None:
                 self.optimizer.prepare_step()  # host work of the next step, before the host read
-            self.last_grad_norm = float(sq.sqrt().item())
+            # the fp32 square root of the fp32 sum, on the host: no launch before the read
+            self.last_grad_norm = float(np.sqrt(np.float32(sq.item())))
             return self.last_grad_norm
+        sq = torch.zeros(1, dtype=torch.float32, device=ps[0].device)
         squares, scaled = [], []
         for p in ps:
             if p.grad is not None:
