@@ -27,6 +27,7 @@
 //                 cycle read on 16 distinct 16-byte bank groups.
 // The tiles of grad_mem are 256 tokens x 192 memory columns (the Gemma-scale 8192 x 1536 output
 // is 256 tiles: one per CU), those of grad_W 256 x 256 (two 5376 x 1536 outputs: 252 tiles).
+// Outputs with fewer such tiles than the part has CUs take smaller tiles (linear_grad_small_kernel).
 // Workgroup ids are remapped so that each XCD's CUs take consecutive tiles, which share rows
 // of A in that XCD's L2. Epilogue: each wave stages its bf16 tile in LDS and writes whole
 // 16-byte row chunks.
@@ -393,21 +394,236 @@ __global__ __launch_bounds__(kThreads, 1) void linear_grad_kernel(const LgArgs a
     }
 }
 
+// ---- small outputs: tiles that fill the part -------------------------------------------------------
+// The same products on 64 BR x 64 BS tiles for outputs of fewer 256-wide tiles than the part has CUs:
+// there one tile's K loop on a fraction of the CUs is the launch's time. Four waves, 2 x 2 over the
+// tile, 32 BR x 32 BS each; whole slabs of both operands in a ring of RING slots, RING - 1 in flight
+// while one is consumed, one barrier per slab. Two workgroups share a CU, so one's waits run under the
+// other's MFMAs. Row-contiguous units are 64 k-rows of a tile's columns (128 or 256 bytes); the chunk
+// swizzle puts the 4 k-rows x 4 chunks of one LDS cycle on 16 distinct 16-byte bank groups.
+template <int COLS>
+__device__ __forceinline__ int small_swizzle(int kr) {
+    static_assert(COLS == 64 || COLS == 128, "8 or 16 chunks per k-row");
+    return COLS == 128 ? 4 * (kr & 3) : 4 * ((kr >> 1) & 1);
+}
+
+template <int COLS>
+__device__ __forceinline__ uint32_t small_lane_off(int col0, int lane) {  // as rc_lane_off
+    const int i = lane & 15, g = lane >> 4;
+    const int c = col0 + 16 * (g & 1) + 4 * (i & 3);
+    const int kr = 8 * (g >> 1) + (i >> 2);
+    return static_cast<uint32_t>(kr * (2 * COLS) + (((c >> 3) ^ small_swizzle<COLS>(kr)) << 4) + (c & 7) * 2);
+}
+
+template <int COLS>
+__device__ __forceinline__ bf16x8 small_frag(const uint8_t *unit, int ks, uint32_t off) {  // as rc_frag
+    const auto *p = (const __attribute__((address_space(3))) uint8_t *)(unit + off) + ks * 16 * (2 * COLS);
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)(p));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)(p + 4 * (2 * COLS)));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+template <bool A_KC, int BR, int BS, int RING>
+__global__ __launch_bounds__(kThreads) void linear_grad_small_kernel(const LgArgs a) {
+    constexpr int TR = 64 * BR, TS = 64 * BS;
+    constexpr int kUnitA = TR * kSlabBytes;     // TR rows x 128 bytes, or 64 k-rows x 2 TR bytes
+    constexpr int kSlot = (TR + TS) * kSlabBytes;
+    constexpr int kDmaA = TR / 32, kDmaB = TS / 32;  // 1 KiB loads per wave and slab
+    constexpr int kPitch = TS * 2 + 16;         // staged output row
+    static_assert(RING >= 3 && TR * kPitch <= RING * kSlot, "the epilogue stage fits the ring");
+    static_assert((RING - 2) * (kDmaA + kDmaB) <= 63, "vmcnt counts up to 63");
+    __shared__ __attribute__((aligned(16))) uint8_t ring[RING * kSlot];
+
+    const int bid = blockIdx.x;
+    const int logical = (bid % kXcds) * a.per_xcd + bid / kXcds;
+    if (logical >= a.total) return;
+    const int per_problem = a.n_rt * a.n_st;
+    const int prob = logical / per_problem;
+    const int rem = logical - prob * per_problem;
+    const int rt = rem / a.n_st, st = rem - (rem / a.n_st) * a.n_st;
+    const int64_t r0 = static_cast<int64_t>(rt) * TR;
+    const int64_t s0 = static_cast<int64_t>(st) * TS;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave >> 1, ws = wave & 1;
+    const int spq = static_cast<int>(ceil_div(a.K, kSlabK));
+    const int slabs = spq * a.ksegs;
+    const int o1 = min(prob + 1, 1);
+
+    // per-lane load offsets, fixed for the K loop: a k-contiguous load fills 8 rows, a row-contiguous
+    // one 512 / columns k-rows; columns past the matrix read zeros
+    const int64_t lda = a.a[prob].ld, ldb = a.b[prob].ld;
+    uint32_t offa[kDmaA], offb[kDmaB];
+#pragma unroll
+    for (int i = 0; i < kDmaA; ++i) {
+        if constexpr (A_KC) {
+            const int row = (wave * kDmaA + i) * 8 + (lane >> 3);
+            const uint32_t ch = static_cast<uint32_t>((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+            offa[i] = r0 + row < a.R ? static_cast<uint32_t>((r0 + row) * lda * 2) + ch : kOff;
+        } else {
+            constexpr int kChunks = TR / 8;
+            const int kr = (wave * kDmaA + i) * (64 / kChunks) + lane / kChunks;
+            const int64_t col = r0 + 8 * ((lane % kChunks) ^ small_swizzle<TR>(kr));
+            offa[i] = col < a.R ? static_cast<uint32_t>((kr * lda + col) * 2) : kOff;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kDmaB; ++i) {
+        constexpr int kChunks = TS / 8;
+        const int kr = (wave * kDmaB + i) * (64 / kChunks) + lane / kChunks;
+        const int64_t col = s0 + 8 * ((lane % kChunks) ^ small_swizzle<TS>(kr));
+        offb[i] = col < a.S ? static_cast<uint32_t>((kr * ldb + col) * 2) : kOff;
+    }
+    const uint32_t ring_lds = lds_addr(ring);
+    // descriptor of a row-contiguous operand from k-row k0 on: what lies past it reads zeros
+    auto from_row = [](const Operand &o, int64_t k0) {
+        const uint64_t shift = static_cast<uint64_t>(k0 * o.ld * 2);
+        return buffer_rsrc(static_cast<const uint8_t *>(o.base) + shift, o.bytes - static_cast<uint32_t>(shift));
+    };
+    auto issue = [&](int sl) {
+        const int q = sl >= spq ? 1 : 0;
+        const int64_t k0 = static_cast<int64_t>(sl - q * spq) * kSlabK;
+        const Operand &oa = a.a[q ? o1 : prob], &ob = a.b[q ? o1 : prob];
+        const uint32_t slot = ring_lds + static_cast<uint32_t>(sl % RING) * kSlot;
+        const int32x4 ra = A_KC ? buffer_rsrc(oa.base, oa.bytes) : from_row(oa, k0);
+        const int32x4 rb = from_row(ob, k0);
+#pragma unroll
+        for (int i = 0; i < kDmaA; ++i)
+            dma16(ra, __builtin_amdgcn_readfirstlane(slot + static_cast<uint32_t>(wave * kDmaA + i) * 1024u), offa[i],
+                  A_KC ? static_cast<uint32_t>(k0 * 2) : 0u);
+#pragma unroll
+        for (int i = 0; i < kDmaB; ++i)
+            dma16(rb, __builtin_amdgcn_readfirstlane(slot + kUnitA + static_cast<uint32_t>(wave * kDmaB + i) * 1024u),
+                  offb[i], 0u);
+    };
+
+    uint32_t soff[BS], roff[A_KC ? 1 : BR];
+#pragma unroll
+    for (int x = 0; x < BS; ++x) soff[x] = small_lane_off<TS>(ws * 32 * BS + 32 * x, lane);
+    if constexpr (!A_KC) {
+#pragma unroll
+        for (int y = 0; y < BR; ++y) roff[y] = small_lane_off<TR>(wr * 32 * BR + 32 * y, lane);
+    }
+    floatx16 acc[BS][BR];
+#pragma unroll
+    for (int x = 0; x < BS; ++x)
+#pragma unroll
+        for (int y = 0; y < BR; ++y)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[x][y][e] = 0.f;
+
+#pragma unroll
+    for (int sl = 0; sl < RING - 1; ++sl)
+        if (sl < slabs) issue(sl);
+    for (int sl = 0; sl < slabs; ++sl) {
+        // slab sl landed for this wave (later slabs may fly), then for every wave
+        if (sl + RING - 2 < slabs)
+            wait_vmcnt<(RING - 2) * (kDmaA + kDmaB)>();
+        else
+            wait_vmcnt<0>();
+        __syncthreads();
+        // the slot of slab sl - 1 is free: every wave read it before this barrier
+        if (sl + RING - 1 < slabs) issue(sl + RING - 1);
+        const uint8_t *ua = ring + (sl % RING) * kSlot, *ub = ua + kUnitA;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            bf16x8 fs[BS], fr[BR];
+#pragma unroll
+            for (int x = 0; x < BS; ++x) fs[x] = small_frag<TS>(ub, ks, soff[x]);
+#pragma unroll
+            for (int y = 0; y < BR; ++y) {
+                if constexpr (A_KC)
+                    fr[y] = kc_frag(ua, ks, wr * 32 * BR + 32 * y + (lane & 31), lane);
+                else
+                    fr[y] = small_frag<TR>(ua, ks, roff[y]);
+            }
+#pragma unroll
+            for (int x = 0; x < BS; ++x)
+#pragma unroll
+                for (int y = 0; y < BR; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fs[x], fr[y], acc[x][y], 0, 0, 0);
+        }
+    }
+    __syncthreads();  // every wave is done with the ring, and no load is in flight
+
+    // acc[x][y][4 g + e]: row 32 y + (lane & 31), column 32 x + 8 g + 4 (lane >> 5) + e of the wave's part
+#pragma unroll
+    for (int x = 0; x < BS; ++x)
+#pragma unroll
+        for (int y = 0; y < BR; ++y)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                uint32_t w[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    w[h] = static_cast<uint32_t>(float_to_bf16_bits_rne(acc[x][y][4 * g + 2 * h])) |
+                           (static_cast<uint32_t>(float_to_bf16_bits_rne(acc[x][y][4 * g + 2 * h + 1])) << 16);
+                const int row = wr * 32 * BR + 32 * y + (lane & 31);
+                const int col = ws * 32 * BS + 32 * x + 8 * g + 4 * (lane >> 5);
+                *reinterpret_cast<uint2 *>(ring + row * kPitch + col * 2) = make_uint2(w[0], w[1]);
+            }
+    __syncthreads();
+    uint16_t *c = a.c[prob];
+    for (int it = tid; it < TR * (TS / 8); it += kThreads) {
+        const int row = it / (TS / 8), cc = it % (TS / 8);
+        const int64_t rg = r0 + row, sg = s0 + cc * 8;
+        if (rg < a.R && sg < a.S)
+            *as_global(reinterpret_cast<u32x4_v *>(c + rg * a.ldc + sg)) =
+                *reinterpret_cast<const u32x4_v *>(ring + row * kPitch + cc * 16);
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void zero_u16_kernel(uint16_t *p, int64_t n) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     for (int64_t k = i; k < n; k += stride) p[k] = 0;
 }
 
-template <bool A_KC, int TS>
-int launch(LgArgs &args, hipStream_t s) {
-    args.n_rt = static_cast<int>(ceil_div(args.R, kTileR));
-    args.n_st = static_cast<int>(ceil_div(args.S, TS));
+int tiles_of(LgArgs &args, int tr, int ts) {
+    args.n_rt = static_cast<int>(ceil_div(args.R, tr));
+    args.n_st = static_cast<int>(ceil_div(args.S, ts));
     args.total = args.problems * args.n_rt * args.n_st;
     args.per_xcd = static_cast<int>(ceil_div(args.total, kXcds));
+    return args.total;
+}
+
+template <bool A_KC, int BR, int BS, int RING>
+int launch_small(LgArgs &args, hipStream_t s) {
+    tiles_of(args, 64 * BR, 64 * BS);
+    hipLaunchKernelGGL((linear_grad_small_kernel<A_KC, BR, BS, RING>), dim3(static_cast<unsigned>(args.per_xcd * kXcds)),
+                       dim3(kThreads), 0, s, args);
+    return check_launch("me_linear_grads");
+}
+
+template <bool A_KC, int TS>
+int launch_large(LgArgs &args, hipStream_t s) {
+    tiles_of(args, kTileR, TS);
     hipLaunchKernelGGL((linear_grad_kernel<A_KC, TS>), dim3(static_cast<unsigned>(args.per_xcd * kXcds)),
                        dim3(kThreads), 0, s, args);
     return check_launch("me_linear_grads");
+}
+
+// The smallest tiles that all find a place at once (two 64 x 64 or 128 x 64 workgroups per CU, one
+// 128 x 128), else the 256-row tiles, whose K loop does four times the work per byte staged. us, large
+// tiles / the small ones taken, n x model dim x memory dim:
+//   grad_mem  64 x 64: 512 x 1024 x 512 33.7 / 12.1, 2042 x 2048 x 1024 61.9 / 31.7, 1000 x 5376 x 1536
+//             150 / 87; 128 x 64: 4096 x 2048 x 1024 62.9 / 46.1, 8192 x 1024 x 512 35.1 / 25.7; past
+//             both, 3000 x 3584 x 1536 104 against 120 with 128 x 64
+//   grad_W    64 x 64: 512 x 1024 x 512 15.7 / 5.5, 8192 x 1024 x 512 142 / 44; 128 x 128:
+//             2042 x 2048 x 1024 43.7 / 25.4, 8192 x 2048 x 1024 147 / 81.5; past both,
+//             3000 x 3584 x 1536 65.6 against 93.9 with 128 x 128
+constexpr int kCus = 256;
+
+int launch_grad_mem(LgArgs &args, hipStream_t s) {
+    if (tiles_of(args, 64, 64) <= 2 * kCus) return launch_small<true, 1, 1, 4>(args, s);
+    if (tiles_of(args, 128, 64) <= 2 * kCus) return launch_small<true, 2, 1, 3>(args, s);
+    return launch_large<true, 192>(args, s);
+}
+
+int launch_grad_w(LgArgs &args, hipStream_t s) {
+    if (tiles_of(args, 64, 64) <= 2 * kCus) return launch_small<false, 1, 1, 4>(args, s);
+    if (tiles_of(args, 128, 128) <= kCus) return launch_small<false, 2, 2, 4>(args, s);
+    return launch_large<false, 256>(args, s);
 }
 
 bool aligned16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -452,7 +668,7 @@ extern "C" int me_linear_grads(const void *grad_key, const void *grad_value, int
         args.K = model_dim;
         args.ksegs = 2;
         args.problems = 1;
-        const int rc = launch<true, 192>(args, s);
+        const int rc = launch_grad_mem(args, s);
         if (rc != ME_OK) return rc;
     }
     if (!any_w) return ME_OK;
@@ -491,5 +707,5 @@ extern "C" int me_linear_grads(const void *grad_key, const void *grad_value, int
     args.K = n;
     args.ksegs = 1;
     args.problems = p;
-    return launch<false, 256>(args, s);
+    return launch_grad_w(args, s);
 }

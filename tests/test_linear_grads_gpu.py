@@ -60,6 +60,17 @@ def test_linear_grads_small_shapes_float64(n, d, M):
         _check(got, ref, mag, name)
 
 
+# the sizes above make 64 x 64 tiles; these grad_mem tiles of 128 x 64 and of 256 x 192, and grad_W
+# tiles of 128 x 128 and of 256 x 256, each with partial tiles on both sides
+@pytest.mark.parametrize("n,d,M", [(4100, 64, 520), (8200, 64, 712), (200, 2112, 520), (130, 3136, 1288)])
+def test_linear_grads_every_tile_float64(n, d, M):
+    ops_in = _operands(n, d, M, seed=n)
+    d_mem, d_wk, d_wv = ops.linear_grads(*(t.to(DEV) for t in ops_in), True, True, True)
+    refs = _refs(*ops_in, torch.float64, "cpu")
+    for got, (ref, mag), name in zip((d_mem, d_wk, d_wv), refs, ("mem", "w_key", "w_value")):
+        _check(got, ref, mag, name)
+
+
 def test_linear_grads_gemma_scale_fp32_reference():
     n, d, M = 8192, 5376, 1536
     ops_in = _operands(n, d, M, seed=5)
