@@ -24,15 +24,25 @@
 // token count, padding columns and k past mem_dim read as zeros (per-lane offsets past the
 // buffer); nothing outside the real output is stored.
 //
-// bf16: v_mfma_f32_16x16x32_bf16, a slab is 2 k-steps of 32. fp32: v_mfma_f32_16x16x4f32, a slab
-// is 2 k-steps of 16: each lane reads 4 consecutive values and the four MFMAs of the step take
+// bf16: v_mfma_f32_16x16x32_bf16, a slab is 2 k-steps of 32. fp32, few tiles: v_mfma_f32_16x16x4f32, a
+// slab is 2 k-steps of 16: each lane reads 4 consecutive values and the four MFMAs of the step take
 // component i of every lane (the sum runs over the same k in a permuted order in both operands).
+// fp32, many tiles: the fp32 matrix rate (157 TFLOP/s) bounds those, so a slab is one k-step of 32 on the
+// bf16 matrix cores. Each value is split exactly into three bf16 parts as its fragment is read (11
+// vector instructions per pair), and six of the nine products of the parts are accumulated in fp32;
+// the other three are below 2^-26 of each term. 2-norm error against 64 bits, normal values, memory dim
+// 512 / 1024 / 1536: 3.4e-7 / 4.8e-7 / 6.0e-7 (fp32 MFMAs 4.1e-7 / 5.7e-7 / 7.0e-7); the parts of values under
+// 2^-110 end below the smallest bf16. The splitting and the MFMAs take turns on a SIMD (2048
+// tokens at 1024 x 1024: 61.6 us, 24 of them MFMAs at their full rate): one wave with the next
+// slab's splitting placed between its MFMAs, 16x16x32 or 32x32x16, took as long.
 #include "me_common.h"
 
 namespace me {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef int int32x4 __attribute__((ext_vector_type(4)));
 
@@ -102,8 +112,33 @@ struct Mma<float> {  // a 16-byte fragment is four k values of each lane group: 
     }
 };
 
+// Eight fp32 values of a lane as three bf16 fragments that add up to them exactly: each value rounded to
+// the nearest bf16, then what remains, twice (24 bits of significand in three times 8).
+struct Split {
+    u32x4_v p[3];
+};
+
+__device__ __forceinline__ Split split_of(const u32x4_v &lo, const u32x4_v &hi) {
+    Split s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float x = __uint_as_float(i < 2 ? lo[2 * i] : hi[2 * i - 4]);
+        float y = __uint_as_float(i < 2 ? lo[2 * i + 1] : hi[2 * i - 3]);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            // one v_cvt_pk_bf16_f32 for the pair
+            const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
+            s.p[t][i] = w;
+            x -= __uint_as_float(w << 16);
+            y -= __uint_as_float(w & 0xffff0000u);
+        }
+    }
+    return s;
+}
+
 // T: element type; BA x BB 16-row blocks per wave (tokens x columns); waves 2 x 2; R ring slots.
-template <typename T, int BA, int BB, int R>
+// SPLIT (fp32): the products on the bf16 matrix cores.
+template <typename T, int BA, int BB, int R, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     constexpr int kEs = sizeof(T);
     constexpr int TM = 2 * 16 * BA;               // tokens per tile
@@ -114,6 +149,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     static_assert(kDma % 4 == 0, "each wave issues the same number of loads");
     constexpr int kDmaWave = kDma / 4;
     static_assert(R >= 3 && R * kSlot <= kLdsBytes, "ring must fit in LDS");
+    static_assert(!SPLIT || kEs == 4, "fp32 values are split");
     static_assert((R - 2) * kDmaWave <= 63, "vmcnt counts up to 63");
     constexpr int kStagePitch = TN * kEs + 16;    // epilogue staging row: TN values + pad
     static_assert(TM * kStagePitch <= R * kSlot, "epilogue staging must fit in the ring");
@@ -200,18 +236,68 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
         // the slot of slab sl - 1 is free: every wave read it before this barrier
         if (sl + R - 1 < slabs) issue(sl + R - 1);
         const uint8_t *slot = ring + (sl % R) * kSlot;
+        if constexpr (SPLIT) {  // one k-step of 32: chunks fq and 4 + fq of both operands
+            Split fa[BA], fb[BB];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            u32x4_v fa[BA], fb[BB];
+            for (int i = 0; i < BA; ++i) {
+                const int row = wa * 16 * BA + 16 * i + fr;
+                fa[i] = split_of(frag(slot, row, 0), frag(slot, row, 1));
+            }
 #pragma unroll
-            for (int i = 0; i < BA; ++i) fa[i] = frag(slot, wa * 16 * BA + 16 * i + fr, ks);
+            for (int j = 0; j < BB; ++j) {
+                const int row = TM + wb * 16 * BB + 16 * j + fr;
+                fb[j] = split_of(frag(slot, row, 0), frag(slot, row, 1));
+            }
+            // of the nine products of the parts the three below 2^-26 of the first are left out; the small
+            // ones come first, each over every block before the next: an MFMA waits for its accumulator
+            constexpr int kA[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-            for (int j = 0; j < BB; ++j) fb[j] = frag(slot, TM + wb * 16 * BB + 16 * j + fr, ks);
+            for (int t = 0; t < 6; ++t)
 #pragma unroll
-            for (int i = 0; i < BA; ++i)
+                for (int i = 0; i < BA; ++i)
 #pragma unroll
-                for (int j = 0; j < BB; ++j) Mma<T>::run(acc[i][j], fa[i], fb[j]);
+                    for (int j = 0; j < BB; ++j) Mma<uint16_t>::run(acc[i][j], fa[i].p[kA[t]], fb[j].p[kB[t]]);
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                u32x4_v fa[BA], fb[BB];
+#pragma unroll
+                for (int i = 0; i < BA; ++i) fa[i] = frag(slot, wa * 16 * BA + 16 * i + fr, ks);
+#pragma unroll
+                for (int j = 0; j < BB; ++j) fb[j] = frag(slot, TM + wb * 16 * BB + 16 * j + fr, ks);
+#pragma unroll
+                for (int i = 0; i < BA; ++i)
+#pragma unroll
+                    for (int j = 0; j < BB; ++j) Mma<T>::run(acc[i][j], fa[i], fb[j]);
+            }
         }
+    }
+    if constexpr (SPLIT) {
+        // A value that is not finite has no such parts (its remainder is NaN; that of a value whose
+        // rounding overflows is infinite), so blocks whose sums are not finite are made again from the values themselves, in fp32 MFMAs.
+#pragma unroll
+        for (int i = 0; i < BA; ++i)
+#pragma unroll
+            for (int j = 0; j < BB; ++j) {
+                bool bad = false;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) bad |= (__float_as_uint(acc[i][j][r]) & 0x7f800000u) == 0x7f800000u;
+                if (__any(bad)) {
+                    const int64_t tok = tok0 + wa * 16 * BA + 16 * i + fr;
+                    const int64_t vc = col0 + wb * 16 * BB + 16 * j + fr;
+                    const int64_t jr = vc < a.d_pad ? vc : vc - a.d_pad;
+                    const bool live_t = tok < a.n, live_c = jr < a.d && vc < 2 * a.d_pad;
+                    const float *pt = reinterpret_cast<const float *>(a.mem) + (live_t ? tok : 0) * a.m;
+                    const float *pc = reinterpret_cast<const float *>(vc < a.d_pad ? a.wk : a.wv) + (live_c ? jr : 0) * a.m;
+                    floatx4 sum = floatx4{0.f, 0.f, 0.f, 0.f};
+                    for (int64_t k0 = 0; k0 < a.m; k0 += 4) {  // m % 4 == 0
+                        const float x = live_t ? *as_global(pt + k0 + fq) : 0.f;
+                        const float y = live_c ? *as_global(pc + k0 + fq) : 0.f;
+                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, sum, 0, 0, 0);
+                    }
+                    acc[i][j] = sum;
+                }
+            }
     }
     __syncthreads();  // every wave is done with the ring (and no load is in flight): stage there
 
@@ -230,6 +316,9 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
                     *reinterpret_cast<uint16_t *>(p) = float_to_bf16_bits_rne(acc[i][j][r]);
                 else
                     *reinterpret_cast<float *>(p) = acc[i][j][r];
+                // one store at a time: this compiler has merged two of these into a ds_write2_b32 with a wrong
+                // offset (tiles of 64 fp32 columns: 51 for 204), which the GPU tests of those tiles show
+                asm volatile("" : : : "memory");
             }
     __syncthreads();
     // 16-byte row segments: TM rows x (TN * kEs / 16) segments
@@ -376,14 +465,14 @@ int few(const ProjArgs &a, hipStream_t s) {
     return launch_few<T, 4>(a, s);
 }
 
-template <typename T, int BA, int BB, int R>
+template <typename T, int BA, int BB, int R, bool SPLIT = false>
 int launch(ProjArgs a, hipStream_t s) {
     constexpr int TM = 32 * BA, TN = 32 * BB;
     a.tiles_tok = static_cast<int>(ceil_div(a.n, TM));
     const int tiles_col = static_cast<int>(ceil_div(2 * a.d_pad, TN));
     a.tiles_total = a.tiles_tok * tiles_col;
     a.per_xcd = static_cast<int>(ceil_div(a.tiles_total, kXcds));
-    hipLaunchKernelGGL((proj_kernel<T, BA, BB, R>), dim3(static_cast<unsigned>(a.per_xcd * kXcds)),
+    hipLaunchKernelGGL((proj_kernel<T, BA, BB, R, SPLIT>), dim3(static_cast<unsigned>(a.per_xcd * kXcds)),
                        dim3(kThreads), 0, s, a);
     return check_launch("me_kv_proj");
 }
@@ -436,15 +525,15 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // at 2048 x 1024, 1024 tokens: 24.8, 14.9; 2048: 25.7, 27.1; 8192: 76.7, 107; at 1024 x 512, 2048
     // tokens: 16.9, 10.6). Both were measured against 128 x 192 tiles (512 tokens 29.2 us, 1024: 51.5,
     // 1237: 73.2, 8192: 363), which stay for many tokens of a memory width the first cannot take.
-    // fp32 (model dim 1024, mem dim 1024): small tiles fill the CUs and two workgroups
-    // share one -- up to 768 tokens 32 x 64 (256 tokens 16.7 us against 72.5 with 128 x 128),
-    // up to 1024 32 x 128 (40.9 us), above 64 x 128 with a three-slot ring (2048 tokens 72.3 us
-    // against 74.8, 8192 tokens 276 against 295).
+    // fp32: fp32 MFMAs on 32 x 64 tiles while all of them find a place (us, model dim and memory dim
+    // 1024: 100 tokens 16.3, 18.4 split; 200: 16.9, 26.4; 300: 23.9, 27.0), then split products on 64 x 64
+    // (1000 tokens: 38.5; 40.9 in fp32 on 32 x 128) and on 64 x 128 ones (2048 tokens 61.6; fp32 71.7;
+    // 4096: 119, 140; 777 tokens at 2000 x 512: 32.4, 41.9; 4096 at 2048 x 1536: 344, 409).
     if (n <= kFewTokens && a.slabs <= 48 && 2 * a.d_pad / 16 * n * a.row_bytes <= kFewBytes)
         return dtype == ME_BF16 ? few<uint16_t>(a, s) : few<float>(a, s);
+    constexpr int64_t kCus = 256;
+    auto tiles = [&](int tokens, int cols) { return ceil_div(n, tokens) * ceil_div(2 * a.d_pad, cols); };
     if (dtype == ME_BF16) {
-        constexpr int64_t kCus = 256;
-        auto tiles = [&](int tokens, int cols) { return ceil_div(n, tokens) * ceil_div(2 * a.d_pad, cols); };
         if (tiles(32, 32) <= 2 * kCus) return launch<uint16_t, 1, 1, 6>(a, s);
         if (tiles(64, 64) <= 2 * kCus) return launch<uint16_t, 2, 2, 4>(a, s);
         if (tiles(64, 96) <= 2 * kCus) return launch<uint16_t, 2, 3, 4>(a, s);
@@ -458,7 +547,7 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
         }
         return launch<uint16_t, 2, 4, 3>(a, s);
     }
-    if (n <= 768) return launch<float, 1, 2, 5>(a, s);
-    if (n <= 1024) return launch<float, 1, 4, 4>(a, s);
-    return launch<float, 2, 4, 3>(a, s);
+    if (tiles(32, 64) <= 2 * kCus) return launch<float, 1, 2, 5>(a, s);
+    if (tiles(64, 64) <= 2 * kCus) return launch<float, 2, 2, 4, true>(a, s);
+    return launch<float, 2, 4, 3, true>(a, s);
 }

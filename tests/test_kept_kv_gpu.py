@@ -79,6 +79,56 @@ def test_kv_proj_few_tokens(n, d, m, dtype):
     _check_proj(n, d, m, dtype)
 
 
+# fp32 past the few-token kernel: fp32 MFMAs on tiles of 32 x 64, split products on 64 x 64 and 64 x 128, by
+# the tiles they make; memory rows of whole and partial slabs, columns and tokens that end inside a tile
+@pytest.mark.parametrize("n,d,m", [(65, 264, 1536), (300, 1024, 200), (700, 1032, 96), (1000, 1024, 36), (1025, 1024, 64),
+                                   (2049, 520, 4), (1025, 2056, 200)])
+def test_kv_proj_fp32_tiles(n, d, m):
+    _check_proj(n, d, m, torch.float32)
+
+
+@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1025, 2056)])
+def test_kv_proj_fp32_values_of_any_size(n, d):
+    # rows and columns scaled by 2^-40 .. 2^40: the split is exact at every exponent, so the bound of
+    # _check_proj holds relative to each element's own magnitudes
+    m = 64
+    g = torch.Generator(device=DEV).manual_seed(3)
+    scale = lambda k: 2.0 ** torch.randint(-40, 41, (k, 1), generator=g, device=DEV).float()
+    mem = torch.randn(n, m, generator=g, device=DEV) * scale(n)
+    wk, wv = (torch.randn(d, m, generator=g, device=DEV) * scale(d) for _ in range(2))
+    kv = ops.kv_proj(mem, wk, wv).double()
+    w = torch.cat([wk, wv]).double().t().contiguous()
+    ref, mag = mem.double() @ w, mem.double().abs() @ w.abs()
+    assert bool(((kv - ref).abs() <= 2.0 ** -24 * ref.abs() + (m + 1) * 2.0 ** -24 * mag).all())
+
+
+@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1025, 2056)])
+def test_kv_proj_fp32_infinities_and_nan(n, d):
+    # where a value is infinite or NaN, so is what the products give, and nothing else changes
+    m = 64
+    g = torch.Generator(device=DEV).manual_seed(4)
+    mem = torch.randn(n, m, generator=g, device=DEV)
+    wk, wv = (torch.randn(d, m, generator=g, device=DEV) for _ in range(2))
+    clean = ops.kv_proj(mem, wk, wv)
+    mem[5, 7], mem[n - 1, m - 1], mem[40, 3] = float("inf"), float("nan"), float("-inf")
+    wk[11, 2], wv[d - 1, 0], wv[3] = float("-inf"), float("nan"), 0.0
+    mem[41] = torch.finfo(torch.float32).max
+    kv = ops.kv_proj(mem, wk, wv)
+    w = torch.cat([wk, wv]).double().t().contiguous()
+    ref = mem.double() @ w
+    ref = torch.where(ref.abs() > torch.finfo(torch.float32).max, ref.sign() * float("inf"), ref)
+    near = torch.zeros_like(ref, dtype=torch.bool)
+    near[41] = True  # sums of the largest values may overflow on the way
+    assert bool(((torch.isnan(ref) == torch.isnan(kv)) | near).all())
+    assert bool(((torch.isinf(ref) == torch.isinf(kv)) | near).all())
+    same = torch.isfinite(ref) & ~near
+    err = (kv.double() - ref).abs() <= 1e-4 + 1e-4 * ref.abs()
+    assert bool((err | ~same).all())
+    rows = [i for i in range(n) if i not in (5, 40, 41, n - 1)]
+    cols = [j for j in range(2 * d) if j not in (11, 2 * d - 1, d + 3)]
+    assert (kv[rows][:, cols] - clean[rows][:, cols]).abs().max() <= 1e-4
+
+
 def _make(dtype, d, tables=6, dim=32):
     torch.manual_seed(d)
     eng = MicroEngram(model_dim=d, table_size=257, engram_dim=dim, num_heads=tables // 2, orders=(2, 3),
