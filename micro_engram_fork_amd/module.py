@@ -118,10 +118,13 @@ class _GateResidual(torch.autograd.Function):
         ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv)
         ctx.gate_mode = gate_mode
         ctx.mark_non_differentiable(alpha)
+        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient
         return out, alpha
 
     @staticmethod
     def backward(ctx, grad_out, _grad_alpha):
+        if grad_out is None:
+            return (None,) * len(ctx.needs_input_grad)
         hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv = ctx.saved_tensors
         need = ctx.needs_input_grad
         wk, wv = w_key.detach(), w_value.detach()
@@ -176,10 +179,13 @@ class _GateResidualRows(torch.autograd.Function):
         ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, k, v)
         ctx.gate_mode = gate_mode
         ctx.mark_non_differentiable(alpha)
+        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient
         return out, alpha
 
     @staticmethod
     def backward(ctx, grad_out, _grad_alpha):
+        if grad_out is None:
+            return (None,) * len(ctx.needs_input_grad)
         hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, k, v = ctx.saved_tensors
         need = ctx.needs_input_grad
         wk, wv = w_key.detach(), w_value.detach()
@@ -430,9 +436,10 @@ class MicroEngram(nn.Module):
                 return mem
         return ops.gather(self._stacked_idx(idx), tables)
 
-    def _mem_grad(self, idx):
+    def _mem_grad(self, idx, read=None):
         """The memory vectors [N, n_tables * D] with the tables' gradients attached: the row
-        lookup of rows.py (dense table gradients, or sparse ones for row shards so marked)."""
+        lookup of rows.py (dense table gradients, or sparse ones for row shards so marked).
+        read: instead of the ids, a function of the tables that hashes and reads in one launch."""
         if self.row_shards is not None:
             if self.row_lookup_fn is not None:
                 return self._served_memory(idx)
@@ -446,7 +453,10 @@ class MicroEngram(nn.Module):
             weights = self._table_parameters()
         from .rows import _RowLookup, _table_offsets
 
-        return _RowLookup.apply(self._stacked_idx(idx), _table_offsets(self), *weights)
+        if read is not None and any(w.shape[0] != rows for w, rows in zip(weights, self.table_rows)):
+            # tables of another size than the hash's: ids past a table's end read as zeros there
+            return _RowLookup.apply(read(None), _table_offsets(self), *weights)
+        return _RowLookup.apply(self._stacked_idx(idx) if read is None else read, _table_offsets(self), *weights)
 
     def lookup(self, idx):
         """The table rows for the hashed ids: list of n_tables tensors [*idx shape, D]
@@ -472,7 +482,10 @@ class MicroEngram(nn.Module):
         """True when `lookup` is not this class's own: set on the instance (as the reference's
         tests do, test_zero_order.py:84-88) or overridden by a subclass. inject and forward then
         read the rows through it, as module.py:233 does."""
-        return "lookup" in self.__dict__ or type(self).lookup is not MicroEngram.lookup
+        return self._replaced("lookup")
+
+    def _replaced(self, name):
+        return name in self.__dict__ or getattr(type(self), name) is not getattr(MicroEngram, name)
 
     # -------------------------------------------------------------------------------- inject
     def _needs_grad(self, hidden):
@@ -561,19 +574,40 @@ class MicroEngram(nn.Module):
             return self._gate(hidden, mem.reshape(-1, mem.shape[-1]), keep)
         if not self._needs_grad(hidden):
             return self._gate(hidden, self._mem(idx), keep)
+        return self._inject_grad(hidden, keep, idx)
+
+    def _inject_grad(self, hidden, keep, idx, read=None):
         from .rows import key_plans_after
 
         with key_plans_after():  # the row dedup's key plan is issued behind the gate
-            return self._gate(hidden, self._mem_grad(idx), keep)
+            return self._gate(hidden, self._mem_grad(idx, read), keep)
 
     def forward(self, hidden, input_ids, position_ids=None):
-        """inject(hidden, hash_ids(input_ids, position_ids)) (module.py:263-265); without
-        gradients the hashing and the gather run as one fused kernel (unless `lookup` has been
-        replaced, which then reads the rows)."""
-        if (self._needs_grad(hidden) or self._lookup_replaced()
-                or (self.row_lookup_fn is not None and self.row_shards is not None)):
+        """inject(hidden, hash_ids(input_ids, position_ids)) (module.py:263-265), with the hashing
+        and the row reads as one launch: the fused kernel without gradients, the same one leaving its
+        row ids for the backward with them. Where lookup, hash_ids or inject has been replaced, or a
+        server's lookup reads the rows, forward goes through those."""
+        if self._lookup_replaced() or (self.row_lookup_fn is not None and self.row_shards is not None):
             return self.inject(hidden, self.hash_ids(input_ids.to(hidden.device), position_ids))
-        return self._gate(hidden, self.hashed_memory(input_ids, position_ids, hidden.device), None)
+        if not self._needs_grad(hidden):
+            return self._gate(hidden, self.hashed_memory(input_ids, position_ids, hidden.device), None)
+        if (torch.compiler.is_compiling() or input_ids.numel() == 0 or self._replaced("hash_ids")
+                or self._replaced("inject")):
+            return self.inject(hidden, self.hash_ids(input_ids.to(hidden.device), position_ids))
+        device = hidden.device
+        ids = input_ids.to(device)
+        pos = position_ids.to(device) if position_ids is not None else None
+
+        def read(tables):
+            """(row ids [n_tables, N], memory vectors); the row ids alone without tables."""
+            canon, mults, ident = self._hash_consts(device)
+            consts = (canon, mults, self._table_orders, self.table_rows, int(self.pad_id))
+            if tables is None:
+                return ops.hash_ids(ids, pos, *consts, ident).reshape(len(self.table_rows), -1)
+            mem, idx = ops.hash_gather(ids, pos, *consts, tables, True, ident)
+            return idx.reshape(len(self.table_rows), -1), mem
+
+        return self._inject_grad(hidden, None, None, read)
 
     def hashed_memory(self, input_ids, position_ids=None, device=None):
         """The concatenated memory vectors [B*T, n_tables * D] of every position: hash_ids +

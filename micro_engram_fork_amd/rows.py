@@ -184,7 +184,13 @@ class _RowLookup(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, idx2d, offsets, *shards):
-        mem = ops.gather(idx2d, list(shards))  # no graph is recorded inside forward
+        """idx2d: the row ids [n_tables, N], or a function of the tables that gives (row ids, memory
+        vectors): MicroEngram.forward hashes and reads in one launch (two launches, with the host work of a list of
+        ids between them, kept the GPU waiting before the gate)."""
+        if callable(idx2d):
+            idx2d, mem = idx2d(list(shards))
+        else:
+            mem = ops.gather(idx2d, list(shards))  # no graph is recorded inside forward
         ctx.save_for_backward(idx2d)
         ctx.offsets = offsets
         ctx.shapes = [(s.shape, s.dtype) for s in shards]
