@@ -136,18 +136,17 @@ __device__ __forceinline__ Split split_of(const u32x4_v &lo, const u32x4_v &hi) 
     return s;
 }
 
-// T: element type; BA x BB 16-row blocks per wave (tokens x columns); waves 2 x 2; R ring slots.
+// T: element type; BA x BB 16-row blocks per wave (tokens x columns); WA x 2 waves; R ring slots.
 // SPLIT (fp32): the products on the bf16 matrix cores.
-template <typename T, int BA, int BB, int R, bool SPLIT>
-__global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
+template <typename T, int BA, int BB, int R, bool SPLIT, int WA>
+__global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
     constexpr int kEs = sizeof(T);
-    constexpr int TM = 2 * 16 * BA;               // tokens per tile
+    constexpr int kWaves = 2 * WA, kBlock = 64 * kWaves;
+    constexpr int TM = WA * 16 * BA;              // tokens per tile
     constexpr int TN = 2 * 16 * BB;               // columns per tile
     constexpr int kRows = TM + TN;                // rows per slab: A (tokens) then B (columns)
-    constexpr int kSlot = kRows * kSlab;          // bytes per ring slot
-    constexpr int kDma = kRows / 8;               // 8-row loads per slab
-    static_assert(kDma % 4 == 0, "each wave issues the same number of loads");
-    constexpr int kDmaWave = kDma / 4;
+    constexpr int kDmaWave = (kRows / 8 + kWaves - 1) / kWaves;  // 8-row loads per wave and slab (past kRows: zeros)
+    constexpr int kSlot = kDmaWave * kWaves * 8 * kSlab;         // bytes per ring slot
     static_assert(R >= 3 && R * kSlot <= kLdsBytes, "ring must fit in LDS");
     static_assert(!SPLIT || kEs == 4, "fp32 values are split");
     static_assert((R - 2) * kDmaWave <= 63, "vmcnt counts up to 63");
@@ -162,7 +161,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     const int col_tile = tile / a.tiles_tok;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wa = wave & 1, wb = wave >> 1;      // the wave's quarter of the tile
+    const int wa = wave % WA, wb = wave / WA;     // the wave's part of the tile
     const int64_t tok0 = static_cast<int64_t>(tok_tile) * TM;
     const int64_t col0 = static_cast<int64_t>(col_tile) * TN;
 
@@ -170,7 +169,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     const int32x4 rk = rsrc_of(a.wk, a.w_bytes);
     const int32x4 rv = rsrc_of(a.wv, a.w_bytes);
 
-    // Load i of this wave fills slab rows 8 (4 i + wave) + [0, 8): lane l takes row + l / 8 at
+    // Load i of this wave fills slab rows 8 (kWaves i + wave) + [0, 8): lane l takes row + l / 8 at
     // physical chunk l % 8, i.e. logical chunk (l % 8) ^ ((row >> 1) & 7). A lane's row offset
     // and chunk are fixed for the whole K loop; per slab the k offset is added, and a chunk past
     // the row (k tail), a token past n or a padding column reads past its buffer (zeros).
@@ -178,7 +177,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     int src[kDmaWave];  // 0: mem, 1: W_K, 2: W_V (uniform per load)
 #pragma unroll
     for (int i = 0; i < kDmaWave; ++i) {
-        const int g8 = 8 * (4 * i + wave);         // first slab row of the load (uniform)
+        const int g8 = 8 * (kWaves * i + wave);    // first slab row of the load (uniform)
         const int row = g8 + (lane >> 3);
         chk[i] = static_cast<uint32_t>((lane & 7) ^ ((row >> 1) & 7)) * 16u;
         if (g8 < TM) {
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
             src[i] = vc0 < a.d_pad ? 1 : 2;
             lim[i] = a.w_bytes;
             const int64_t jr = (vc0 < a.d_pad ? vc0 : vc0 - a.d_pad) + (lane >> 3);
-            roff[i] = (jr < a.d && vc0 < 2 * a.d_pad) ? static_cast<uint32_t>(jr) * a.row_bytes : a.w_bytes;
+            roff[i] = (g8 < kRows && jr < a.d && vc0 < 2 * a.d_pad) ? static_cast<uint32_t>(jr) * a.row_bytes : a.w_bytes;
         }
     }
     const uint32_t ring_lds = lds_addr(ring);
@@ -200,7 +199,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
         const uint32_t kb = static_cast<uint32_t>(sl) * kSlab;
 #pragma unroll
         for (int i = 0; i < kDmaWave; ++i) {
-            const uint32_t dst = __builtin_amdgcn_readfirstlane(slot + static_cast<uint32_t>(4 * i + wave) * 1024u);
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(slot + static_cast<uint32_t>(kWaves * i + wave) * 1024u);
             const bool in = roff[i] < lim[i] && chk[i] + kb < a.row_bytes;
             const uint32_t vo = in ? roff[i] + chk[i] + kb : lim[i];
             dma16(src[i] == 0 ? rm : (src[i] == 1 ? rk : rv), dst, vo);
@@ -325,7 +324,7 @@ __global__ __launch_bounds__(kThreads) void proj_kernel(const ProjArgs a) {
     constexpr int kSegs = TN * kEs / 16;
     constexpr int kPerSeg = 16 / kEs;
     const int64_t stride = 2 * a.d;
-    for (int it = threadIdx.x; it < TM * kSegs; it += kThreads) {
+    for (int it = threadIdx.x; it < TM * kSegs; it += kBlock) {
         const int row = it / kSegs;
         const int seg = it % kSegs;
         const int64_t tok = tok0 + row;
@@ -465,15 +464,15 @@ int few(const ProjArgs &a, hipStream_t s) {
     return launch_few<T, 4>(a, s);
 }
 
-template <typename T, int BA, int BB, int R, bool SPLIT = false>
+template <typename T, int BA, int BB, int R, bool SPLIT = false, int WA = 2>
 int launch(ProjArgs a, hipStream_t s) {
-    constexpr int TM = 32 * BA, TN = 32 * BB;
+    constexpr int TM = 16 * WA * BA, TN = 32 * BB;
     a.tiles_tok = static_cast<int>(ceil_div(a.n, TM));
     const int tiles_col = static_cast<int>(ceil_div(2 * a.d_pad, TN));
     a.tiles_total = a.tiles_tok * tiles_col;
     a.per_xcd = static_cast<int>(ceil_div(a.tiles_total, kXcds));
-    hipLaunchKernelGGL((proj_kernel<T, BA, BB, R, SPLIT>), dim3(static_cast<unsigned>(a.per_xcd * kXcds)),
-                       dim3(kThreads), 0, s, a);
+    hipLaunchKernelGGL((proj_kernel<T, BA, BB, R, SPLIT, WA>), dim3(static_cast<unsigned>(a.per_xcd * kXcds)),
+                       dim3(128 * WA), 0, s, a);
     return check_launch("me_kv_proj");
 }
 
@@ -516,8 +515,14 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // smallest tile whose tiles all find a place at once, two workgroups per CU: 32 x 32 with six slots of
     // 128-byte slabs (19 tokens: 9.2 us; 10.4 with 32 x 96 and four slots; at 2048 x 1024, 128
     // tokens: 6.9, 8.9), 64 x 64 with four (192 tokens: 13.2; 15.6 with 64 x 96; at 3584 x 1536, 256
-    // tokens: 12.7, 15.4), 64 x 96 with four (256 tokens: 16.0; 64 x 64 20.3, 128 x 96 17.6). Larger
-    // batches take the gate's 256 x 224 tiles (one workgroup per CU, a matrix core's worth of work per barrier)
+    // tokens: 12.7, 15.4), 64 x 96 with four (256 tokens: 16.0; 64 x 64 20.3, 128 x 96 17.6, with eight
+    // waves 14.8 by itself but 0.2 us more in a decode step). Tiles of one round, one to a CU, take eight
+    // waves, two per SIMD as two smaller workgroups are, with fewer bytes for the same outputs: 64 x 64 with
+    // six slots (48 tokens: 9.8, 10.5 with four waves, the decode step 24.6 -> 23.7; at 2048 x 1024, 256
+    // tokens: 7.8, 8.2), 256 x 96 (512 tokens: 24.4, 29.1 in 64 x 128; the decode step of 500 tokens 46.7 ->
+    // 42.8) and 256 x 128 with three (700 tokens: 28.2, 33.6; at 3584 x 1536, 1024 tokens: 27.9, 33.8; at
+    // 2048 x 1024, 2042 tokens: 22.2, 25.5). Larger batches take the gate's 256 x 224 tiles (one
+    // workgroup per CU, a matrix core's worth of work per barrier)
     // or 64 x 128 ones (three slots, two workgroups per CU), whichever needs the less time for the
     // whole rounds its tiles make on 256 CUs: a round of the first takes about 7 us and 1.25 us per
     // slab, 256 tiles of the second 1.2 us and 0.33 us per slab, but never under 1.6 such (512
@@ -535,8 +540,13 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     auto tiles = [&](int tokens, int cols) { return ceil_div(n, tokens) * ceil_div(2 * a.d_pad, cols); };
     if (dtype == ME_BF16) {
         if (tiles(32, 32) <= 2 * kCus) return launch<uint16_t, 1, 1, 6>(a, s);
+        if (tiles(64, 64) <= kCus) return launch<uint16_t, 1, 2, 6, false, 4>(a, s);
         if (tiles(64, 64) <= 2 * kCus) return launch<uint16_t, 2, 2, 4>(a, s);
         if (tiles(64, 96) <= 2 * kCus) return launch<uint16_t, 2, 3, 4>(a, s);
+        if (tiles(64, 128) > 2 * kCus) {  // three rounds and more of those below
+            if (tiles(256, 96) <= kCus) return launch<uint16_t, 4, 3, 3, false, 4>(a, s);
+            if (tiles(256, 128) <= kCus) return launch<uint16_t, 4, 4, 3, false, 4>(a, s);
+        }
         const float small = static_cast<float>(ceil_div(tiles(64, 128), kCus));
         if (a.row_bytes % kSlab == 0 && a.slabs >= 3 && n * model_dim * 4 < (int64_t{1} << 31)) {
             const float large = static_cast<float>(ceil_div(ceil_div(n, 256) * 2 * ceil_div(model_dim, 224), kCus));

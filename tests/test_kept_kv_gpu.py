@@ -62,9 +62,9 @@ def _check_proj(n, d, m, dtype):
 
 
 # token counts around the switches between the projection's tiles (by the tiles they make: 32 x 32,
-# 64 x 64, 64 x 96, then 64 x 128 or 256 x 224) and memory widths of whole and partial slabs
+# 64 x 64, 64 x 96, 256 x 96, 256 x 128, then 64 x 128 or 256 x 224) and memory widths of whole and partial slabs
 @pytest.mark.parametrize("n", [64, 65, 192, 193, 256, 257, 512, 513, 768, 1025])
-@pytest.mark.parametrize("d,m", [(5376, 192), (264, 1536), (2048, 200)])
+@pytest.mark.parametrize("d,m", [(5376, 192), (264, 1536), (2048, 200), (5320, 136)])
 def test_kv_proj_tiles(n, d, m):
     _check_proj(n, d, m, torch.bfloat16)
 
