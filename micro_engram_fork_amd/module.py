@@ -109,9 +109,8 @@ class _GateResidual(torch.autograd.Function):
         k = None if k_delta is None else k_delta.detach()
         kv = None
         if keep_kv:
-            d = hidden.shape[-1]
-            kv = ops.kv_proj(mem, w_key.detach(), w_value.detach())
-            out, alpha, stats = ops.gate_rows(hidden, kv[:, :d], kv[:, d:], q, k, gate_mode, keep, True, True)
+            out, alpha, stats, kv = ops.gate_residual_rows(hidden, mem, w_key.detach(), w_value.detach(), q, k,
+                                                           gate_mode, keep, True, True, True)
         else:
             out, alpha, stats = ops.gate_residual(hidden, mem, w_key.detach(), w_value.detach(), q, k,
                                                   gate_mode, keep, True, True)

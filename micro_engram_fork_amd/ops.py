@@ -449,12 +449,15 @@ def prefers_rows(n, model_dim, mem_dim):
     return proj + 2.5 + n * model_dim * 8 / 5.3e6 < -(-tiles // 256) * (25 + 2.2 * slabs)
 
 
-def _kv_rows(k, v, d):
-    """(K rows, V rows, their row stride in elements) for the row kernels: [N, d] tensors as they are
-    when their rows are contiguous and one stride apart (the halves of kv_proj's [N, 2d]), else
+def _kv_rows(k, v, n, d):
+    """(K rows, V rows, their row stride in elements) for the row kernels: [n, d] tensors as they are
+    when their rows are contiguous and one stride apart (the halves of kv_proj's [n, 2d]), else
     contiguous copies."""
     if k.dtype != v.dtype:
         raise ValueError("[micro_engram] K and V rows must share one dtype")
+    if not k.numel() == v.numel() == n * d:
+        raise ValueError(f"[micro_engram] K rows {tuple(k.shape)} and V rows {tuple(v.shape)} do not match "
+                         f"{n} tokens of {d} columns")
     k, v = k.reshape(-1, d), v.reshape(-1, d)
     if k.stride(1) == v.stride(1) == 1 and k.stride(0) == v.stride(0) >= d:
         return k, v, k.stride(0)
@@ -472,10 +475,8 @@ def gate_rows(hidden: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     d = hidden.shape[-1]
     x = hidden.reshape(-1, d).contiguous()
     N = x.shape[0]
-    k, v, kv_stride = _kv_rows(k, v, d)
-    if k.shape[0] != N:
-        raise ValueError(f"[micro_engram] K/V rows {tuple(k.shape)} do not match {N} tokens")
-    q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode)
+    k, v, kv_stride = _kv_rows(k, v, N, d)
+    q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode, d)
     keep_u8 = _keep_u8(keep, N)
     out = torch.empty_like(x)
     alpha = torch.empty(N, dtype=torch.float32, device=dev) if with_alpha else None
@@ -521,12 +522,14 @@ def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Te
     d = hidden.shape[-1]
     x = hidden.reshape(-1, d).contiguous()
     N = x.shape[0]
-    k, v, kv_stride = _kv_rows(k, v, d)
+    k, v, kv_stride = _kv_rows(k, v, N, d)
     g = grad_out.reshape(-1, d).to(x.dtype).contiguous()
+    if g.shape[0] != N:
+        raise ValueError(f"[micro_engram] the output's gradient {tuple(grad_out.shape)} does not match {N} tokens")
     stats = stats.contiguous()
     if tuple(stats.shape) != (N, 4) or stats.dtype != torch.float32:
         raise ValueError(f"[micro_engram] stats must be fp32 [{N}, 4], got {tuple(stats.shape)}")
-    q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode)
+    q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode, d)
     keep_u8 = _keep_u8(keep, N)
     grad_hidden = torch.empty_like(x)
     grad_k = torch.empty((N, d), dtype=k.dtype, device=dev)
@@ -551,12 +554,15 @@ def _(grad_out, hidden, k, v, q_scale_delta, k_scale_delta, gate_mode, keep, sta
             hidden.new_empty((nd,), dtype=torch.float32), hidden.new_empty((nd,), dtype=torch.float32)]
 
 
-def _scales(q_scale_delta, k_scale_delta, gate_mode):
+def _scales(q_scale_delta, k_scale_delta, gate_mode, d):
     """(q delta, k delta, dtype code) for the row kernels; (None, None, 0) for the scalar gate."""
     if gate_mode != _lib.ME_GATE_SCALAR_SQRT:
         return None, None, 0
     if q_scale_delta is None or k_scale_delta is None:
         raise ValueError("[micro_engram] the scalar_sqrt gate needs q_scale and k_scale")
+    if not q_scale_delta.numel() == k_scale_delta.numel() == d:
+        raise ValueError(f"[micro_engram] scales {tuple(q_scale_delta.shape)}, {tuple(k_scale_delta.shape)} do not "
+                         f"match {d} columns")
     q, k = q_scale_delta.contiguous(), k_scale_delta.contiguous()
     if q.dtype != k.dtype:
         k = k.to(q.dtype)
@@ -578,10 +584,11 @@ def gate_residual_rows(hidden: torch.Tensor, mem: torch.Tensor, w_key: torch.Ten
                        w_value: torch.Tensor, q_scale_delta: Optional[torch.Tensor],
                        k_scale_delta: Optional[torch.Tensor], gate_mode: int,
                        keep: Optional[torch.Tensor], with_alpha: bool,
-                       with_stats: bool = False) -> List[torch.Tensor]:
-    """gate_residual for few tokens: [K | V] from me_kv_proj (K and V rounded to mem's dtype, as
+                       with_stats: bool = False, with_kv: bool = False) -> List[torch.Tensor]:
+    """gate_residual as two kernels: [K | V] from me_kv_proj (K and V rounded to mem's dtype, as
     the two nn.Linear calls of module.py:245, 254 give them), then the gate and the residual add
-    in me_gate_rows."""
+    in me_gate_rows. with_kv: [K | V] [N, 2d] comes last in the result (a training forward keeps
+    it for gate_rows_backward)."""
     dev = require_gpu(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, keep)
     x, mem, w_key, w_value, q_scale_delta, k_scale_delta, scale_code, keep_u8, N, d, M = \
         _gate_operands(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, gate_mode, keep)
@@ -601,18 +608,22 @@ def gate_residual_rows(hidden: torch.Tensor, mem: torch.Tensor, w_key: torch.Ten
         res.append(alpha)
     if with_stats:
         res.append(stats)
+    if with_kv:
+        res.append(kv)
     return res
 
 
 @gate_residual_rows.register_fake
 def _(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, gate_mode, keep, with_alpha,
-      with_stats=False):
+      with_stats=False, with_kv=False):
     n = hidden.numel() // hidden.shape[-1]
     res = [torch.empty_like(hidden)]
     if with_alpha:
         res.append(hidden.new_empty((n,), dtype=torch.float32))
     if with_stats:
         res.append(hidden.new_empty((n, 4), dtype=torch.float32))
+    if with_kv:
+        res.append(mem.new_empty((n, 2 * hidden.shape[-1])))
     return res
 
 

@@ -1,0 +1,69 @@
+"""Calls that do not fit are refused before any kernel is launched: the ops' checks run here on CPU tensors
+with the launches recorded instead of made."""
+import pytest
+import torch
+
+from micro_engram_fork_amd import MicroEngram, ops
+from micro_engram_fork_amd._lib import ME_GATE_SCALAR, ME_GATE_SCALAR_SQRT
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    """The names of the library calls made, none of which reaches the library."""
+    seen = []
+    monkeypatch.setattr(ops, "require_gpu", lambda *tensors: torch.device("cpu"))
+    monkeypatch.setattr(ops, "stream_of", lambda device: 0)
+    monkeypatch.setattr(ops, "call", lambda name, *args: seen.append(name))
+    cached = [f for f in vars(ops).values() if hasattr(f, "cache_clear")]  # workspace sizes: none was computed here
+    for f in cached:
+        f.cache_clear()
+    yield seen
+    for f in cached:
+        f.cache_clear()
+
+
+def _engram(d, dtype=torch.float32, gate="scalar_sqrt", **kw):
+    kw = dict(dict(table_size=97, engram_dim=8, num_heads=2, orders=(2, 3), vocab_size=500), **kw)
+    return MicroEngram(d, gate=gate, **kw).to(dtype).train()
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("gate", ["scalar", "scalar_sqrt"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width", [64, 96, 120, 192])
+def test_hidden_of_another_width_is_refused(launches, width, dtype, gate, grad):
+    eng = _engram(128, dtype, gate)
+    hidden = torch.zeros(48, width, dtype=dtype)
+    mem = torch.zeros(48, 32, dtype=dtype, requires_grad=grad)
+    with torch.set_grad_enabled(grad), pytest.raises(ValueError, match="does not match"):
+        eng.gate_residual(hidden, mem)
+    assert launches == []
+    with torch.set_grad_enabled(grad), pytest.raises(ValueError, match="does not match"):
+        eng.gate_residual(torch.zeros(47, 128, dtype=dtype), mem)  # another number of tokens
+    assert launches == []
+    with torch.set_grad_enabled(grad):
+        eng.gate_residual(torch.zeros(48, 128, dtype=dtype), mem)
+    assert launches == ["me_kv_proj", "me_gate_rows"]
+
+
+def test_row_kernels_refuse_rows_that_do_not_fit(launches):
+    n, d = 48, 64
+    x, stats = torch.zeros(n, d), torch.zeros(n, 4)
+    k, q = torch.zeros(n, d), torch.zeros(d)
+    both = [lambda k, v, q, s: ops.gate_rows(x, k, v, q, s, ME_GATE_SCALAR_SQRT, None, True),
+            lambda k, v, q, s: ops.gate_rows_backward(x, x, k, v, q, s, ME_GATE_SCALAR_SQRT, None, stats)]
+    wide = torch.zeros(n, 4 * d)
+    for call in both:
+        for kk, vv in ((k, wide[:, d:]), (wide[:, :d], wide[:, 2 * d:]), (k, k[:16]), (k[:16], k), (k[:, :32], k)):
+            with pytest.raises(ValueError, match="do not match"):
+                call(kk, vv, q, q)
+        for qq, ss in ((q[:32], q), (q, q[:32]), (torch.zeros(2 * d), q)):
+            with pytest.raises(ValueError, match="do not match"):
+                call(k, k, qq, ss)
+    with pytest.raises(ValueError, match="does not match"):
+        ops.gate_rows_backward(x[:16], x, k, k, None, None, ME_GATE_SCALAR, None, stats)
+    assert launches == []
+    for call in both:  # halves of one buffer, and rows of any shape that holds n rows of d
+        call(wide[:, :d], wide[:, d:2 * d], q, q)
+        call(k.view(4, 12, d), k, q, q)
+    assert launches == ["me_gate_rows"] * 2 + ["me_gate_rows_backward_workspace_size"] + ["me_gate_rows_backward"] * 2
