@@ -145,6 +145,8 @@ def _table_args(table_orders, table_rows):
 @functools.lru_cache(maxsize=64)
 def _table_args_of(table_orders, table_rows):
     # ctypes arrays the kernels only read: one per distinct table layout
+    if len(table_orders) != len(table_rows):
+        raise ValueError(f"[micro_engram] {len(table_orders)} table orders for {len(table_rows)} row counts")
     return len(table_orders), i32_array(list(table_orders)), i64_array(list(table_rows))
 
 
@@ -230,6 +232,13 @@ def _tables_arg_checked(tables):
     return ptr_array([t.data_ptr() for t in tables]), i64_array([t.shape[0] for t in tables]), dim
 
 
+def _hashed_tables_arg(tables, n_tables):
+    """_tables_arg of the tables that the row ids of n_tables hashes index."""
+    if len(tables) != n_tables:
+        raise ValueError(f"[micro_engram] {len(tables)} tables for the row ids of {n_tables}")
+    return _tables_arg(tables)
+
+
 @_custom_op("gather")
 def gather(idx: torch.Tensor, tables: List[torch.Tensor]) -> torch.Tensor:
     """mem [N, n_tables * D] from row ids int64 [n_tables, N] (module.py:146-154, 233; rows
@@ -264,7 +273,7 @@ def hash_gather(input_ids: torch.Tensor, position_ids: Optional[torch.Tensor], c
     B, T = ids.shape
     pos, pstride = _pos_arg(position_ids, B, T)
     nt, orders, rows = _table_args(table_orders, table_rows)
-    ptrs, _rows, dim = _tables_arg(tables)
+    ptrs, _rows, dim = _hashed_tables_arg(tables, nt)
     mem = torch.empty((B * T, nt * dim), dtype=tables[0].dtype, device=dev)
     idx = torch.empty((nt, B, T), dtype=torch.int64, device=dev) if with_idx else None
     call("me_hash_gather", ids.data_ptr(), dtype_code(ids), B, T, _p(pos),
@@ -294,7 +303,7 @@ def hash_prev_gather(ids: torch.Tensor, canon: torch.Tensor, mults: torch.Tensor
     ids = _prev_ids(ids)
     N, W = ids.shape
     nt, orders, rows = _table_args(table_orders, table_rows)
-    ptrs, _rows, dim = _tables_arg(tables)
+    ptrs, _rows, dim = _hashed_tables_arg(tables, nt)
     mem = torch.empty((N, nt * dim), dtype=tables[0].dtype, device=dev)
     idx = torch.empty((nt, N), dtype=torch.int64, device=dev) if with_idx else None
     call("me_hash_prev_gather", ids.data_ptr(), dtype_code(ids), N, W, ids.stride(0) if N else W,

@@ -67,3 +67,20 @@ def test_row_kernels_refuse_rows_that_do_not_fit(launches):
         call(wide[:, :d], wide[:, d:2 * d], q, q)
         call(k.view(4, 12, d), k, q, q)
     assert launches == ["me_gate_rows"] * 2 + ["me_gate_rows_backward_workspace_size"] + ["me_gate_rows_backward"] * 2
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("tables", [3, 5])
+def test_a_table_count_other_than_the_hashes_is_refused(launches, tables, grad):
+    # the fused reads take the tables' addresses from a host array as long as the hash's table list
+    eng = _engram(64)
+    rows = [eng.tables[k % 4] for k in range(tables)]
+    eng.tables = torch.nn.ModuleList(rows)
+    hidden, ids = torch.zeros(1, 6, 64), torch.zeros(1, 6, dtype=torch.long)
+    with torch.set_grad_enabled(grad), pytest.raises(ValueError, match="tables for the row ids"):
+        eng(hidden, ids)
+    with torch.no_grad(), pytest.raises(ValueError, match="tables for the row ids"):
+        eng.hash_prev(torch.zeros(6, 3, dtype=torch.long))
+    with pytest.raises(ValueError, match="table orders"):
+        ops.hash_ids(ids, None, eng.canon, eng.mults, eng._table_orders, eng.table_rows[:3], 0)
+    assert launches == []
