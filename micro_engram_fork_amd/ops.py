@@ -210,8 +210,8 @@ _TABLES_ARGS = {}
 
 
 def _tables_arg(tables: Sequence[torch.Tensor]):
-    """(pointer array, row counts, row width) of the tables, checked: kept per (address, shape,
-    strides, dtype) of every table, which fix all three (the arrays are only read)."""
+    """(pointer array, row count array, row width, row counts) of the tables, checked: kept per (address,
+    shape, strides, dtype) of every table, which fix them all (the arrays are only read)."""
     key = tuple((t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tables)
     hit = _TABLES_ARGS.get(key)
     if hit is None:
@@ -229,14 +229,19 @@ def _tables_arg_checked(tables):
             raise ValueError("[micro_engram] tables must be 2-D with one row width and dtype")
         if not t.is_contiguous():
             raise ValueError("[micro_engram] tables must be contiguous")
-    return ptr_array([t.data_ptr() for t in tables]), i64_array([t.shape[0] for t in tables]), dim
+    rows = tuple(int(t.shape[0]) for t in tables)
+    return ptr_array([t.data_ptr() for t in tables]), i64_array(list(rows)), dim, rows
 
 
-def _hashed_tables_arg(tables, n_tables):
-    """_tables_arg of the tables that the row ids of n_tables hashes index."""
-    if len(tables) != n_tables:
-        raise ValueError(f"[micro_engram] {len(tables)} tables for the row ids of {n_tables}")
-    return _tables_arg(tables)
+def _hashed_tables_arg(tables, table_rows):
+    """(pointer array, row width) of the tables that row ids below table_rows[k] index, or (None, row
+    width) where a table has fewer rows than that: the fused reads do not look for a table's end."""
+    if len(tables) != len(table_rows):
+        raise ValueError(f"[micro_engram] {len(tables)} tables for the row ids of {len(table_rows)}")
+    ptrs, _array, dim, rows = _tables_arg(tables)
+    if rows != tuple(table_rows) and any(have < want for have, want in zip(rows, table_rows)):
+        return None, dim
+    return ptrs, dim
 
 
 @_custom_op("gather")
@@ -248,7 +253,7 @@ def gather(idx: torch.Tensor, tables: List[torch.Tensor]) -> torch.Tensor:
         raise ValueError("[micro_engram] idx must be int64 [n_tables, N]")
     if idx.stride(1) != 1:
         idx = idx.contiguous()
-    ptrs, rows, dim = _tables_arg(tables)
+    ptrs, rows, dim, _ = _tables_arg(tables)
     N = idx.shape[1]
     mem = torch.empty((N, len(tables) * dim), dtype=tables[0].dtype, device=dev)
     call("me_gather", idx.data_ptr(), idx.stride(0) if len(tables) > 1 else N, N, len(tables),
@@ -267,13 +272,18 @@ def hash_gather(input_ids: torch.Tensor, position_ids: Optional[torch.Tensor], c
                 tables: List[torch.Tensor], with_idx: bool,
                 identity_canon: bool = False) -> List[torch.Tensor]:
     """[mem [B*T, n_tables*D]] or [mem, idx [n_tables, B, T]]: hash_ids + lookup + cat in one
-    kernel (module.py:263-265)."""
+    kernel (module.py:263-265); in two where a table ends before its row ids do (they then read
+    as zeros, as in gather)."""
     dev = require_gpu(input_ids, position_ids, canon, mults, *tables)
     ids = _ids2d(input_ids)
     B, T = ids.shape
     pos, pstride = _pos_arg(position_ids, B, T)
     nt, orders, rows = _table_args(table_orders, table_rows)
-    ptrs, _rows, dim = _hashed_tables_arg(tables, nt)
+    ptrs, dim = _hashed_tables_arg(tables, table_rows)
+    if ptrs is None:
+        idx = hash_ids(ids, pos, canon, mults, table_orders, table_rows, pad_id, identity_canon)
+        mem = gather(idx.reshape(nt, B * T), tables)
+        return [mem, idx] if with_idx else [mem]
     mem = torch.empty((B * T, nt * dim), dtype=tables[0].dtype, device=dev)
     idx = torch.empty((nt, B, T), dtype=torch.int64, device=dev) if with_idx else None
     call("me_hash_gather", ids.data_ptr(), dtype_code(ids), B, T, _p(pos),
@@ -298,12 +308,17 @@ def hash_prev_gather(ids: torch.Tensor, canon: torch.Tensor, mults: torch.Tensor
                      table_orders: List[int], table_rows: List[int], pad_id: int,
                      tables: List[torch.Tensor], with_idx: bool,
                      identity_canon: bool = False) -> List[torch.Tensor]:
-    """[mem [N, n_tables*D]] or [mem, idx [n_tables, N]]: hash_prev + lookup in one kernel."""
+    """[mem [N, n_tables*D]] or [mem, idx [n_tables, N]]: hash_prev + lookup in one kernel, or in two as
+    hash_gather."""
     dev = require_gpu(ids, canon, mults, *tables)
     ids = _prev_ids(ids)
     N, W = ids.shape
     nt, orders, rows = _table_args(table_orders, table_rows)
-    ptrs, _rows, dim = _hashed_tables_arg(tables, nt)
+    ptrs, dim = _hashed_tables_arg(tables, table_rows)
+    if ptrs is None:
+        idx = hash_prev(ids, canon, mults, table_orders, table_rows, pad_id, identity_canon)
+        mem = gather(idx, tables)
+        return [mem, idx] if with_idx else [mem]
     mem = torch.empty((N, nt * dim), dtype=tables[0].dtype, device=dev)
     idx = torch.empty((nt, N), dtype=torch.int64, device=dev) if with_idx else None
     call("me_hash_prev_gather", ids.data_ptr(), dtype_code(ids), N, W, ids.stride(0) if N else W,

@@ -84,3 +84,20 @@ def test_a_table_count_other_than_the_hashes_is_refused(launches, tables, grad):
     with pytest.raises(ValueError, match="table orders"):
         ops.hash_ids(ids, None, eng.canon, eng.mults, eng._table_orders, eng.table_rows[:3], 0)
     assert launches == []
+
+
+def test_a_table_that_ends_before_its_row_ids_is_read_by_the_gather(launches):
+    # the fused reads take every row id below the hash's row count to be in the table; the gather looks
+    eng = _engram(64).eval()
+    eng.tables[2] = torch.nn.Embedding(50, 8)
+    ids = torch.zeros(1, 6, dtype=torch.long)
+    with torch.no_grad():
+        eng.hashed_memory(ids)
+        eng.hash_prev(torch.zeros(6, 3, dtype=torch.long))
+    assert launches == ["me_hash_ngrams", "me_gather", "me_hash_prev", "me_gather"]
+    launches.clear()
+    eng.tables[2] = torch.nn.Embedding(150, 8)
+    with torch.no_grad():
+        eng.hashed_memory(ids)
+        eng.hash_prev(torch.zeros(6, 3, dtype=torch.long))
+    assert launches == ["me_hash_gather", "me_hash_prev_gather"]

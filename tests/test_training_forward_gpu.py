@@ -69,3 +69,20 @@ def test_replaced_methods_and_table_sizes_keep_their_route():
     idx = eng.hash_ids(ids)
     assert torch.equal(eng(hidden, ids), eng.inject(hidden, idx))
     assert torch.equal(eng(hidden[:, :0], ids[:, :0]), hidden[:, :0])
+
+
+def test_missing_rows_of_a_smaller_table_are_zeros_without_gradients():
+    # the prefill and the decode step, whose fused reads do not look for a table's end
+    eng = _make().eval()
+    rows = eng.tables[1].weight.detach()[:200].clone()
+    eng.tables[1] = torch.nn.Embedding(200, 16, _weight=rows).to(DEV)
+    ids = torch.randint(0, 500, (1, 64), device=DEV)
+    hidden = torch.randn(1, 64, 64, device=DEV).bfloat16()
+    idx = eng.hash_ids(ids)[1].reshape(-1)
+    want = torch.where((idx < 200)[:, None], rows[idx.clamp(max=199)], torch.zeros((), dtype=rows.dtype, device=DEV))
+    assert bool((idx >= 200).any())
+    with torch.no_grad():
+        assert torch.equal(eng.hashed_memory(ids)[:, 16:32], want)
+        prev = torch.stack([ids[0].roll(k) for k in range(3)], dim=1)
+        read = eng.hash_prev(prev)
+        assert torch.equal(eng.inject(hidden, read), eng.inject(hidden, [i.clone() for i in read]))
