@@ -534,6 +534,12 @@ def gate_rows_backward_workspace_bytes(n, d):
     return size.value
 
 
+def _wide_rows(t, d):
+    """t on a 16-byte boundary (a copy if need be) where rows of d columns let the row kernels make
+    16-byte accesses; one column at a time costs them more than the copy."""
+    return t if t is None or d % 8 or _aligned(t) else t.clone()
+
+
 @_custom_op("gate_rows_backward")
 def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Tensor,
                        v: torch.Tensor, q_scale_delta: Optional[torch.Tensor],
@@ -554,6 +560,7 @@ def gate_rows_backward(grad_out: torch.Tensor, hidden: torch.Tensor, k: torch.Te
     if tuple(stats.shape) != (N, 4) or stats.dtype != torch.float32:
         raise ValueError(f"[micro_engram] stats must be fp32 [{N}, 4], got {tuple(stats.shape)}")
     q_scale_delta, k_scale_delta, scale_code = _scales(q_scale_delta, k_scale_delta, gate_mode, d)
+    x, g, q_scale_delta, k_scale_delta = (_wide_rows(t, d) for t in (x, g, q_scale_delta, k_scale_delta))
     keep_u8 = _keep_u8(keep, N)
     grad_hidden = torch.empty_like(x)
     grad_k = torch.empty((N, d), dtype=k.dtype, device=dev)

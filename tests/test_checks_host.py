@@ -101,3 +101,28 @@ def test_a_table_that_ends_before_its_row_ids_is_read_by_the_gather(launches):
         eng.hashed_memory(ids)
         eng.hash_prev(torch.zeros(6, 3, dtype=torch.long))
     assert launches == ["me_hash_gather", "me_hash_prev_gather"]
+
+
+def test_unaligned_operands_with_gradients_are_copied_once(monkeypatch):
+    # hidden, the output's gradient and the scales on odd addresses: both row kernels get copies they can read
+    # 16 bytes at a time (else they take one column per lane)
+    calls = {}
+    monkeypatch.setattr(ops, "require_gpu", lambda *tensors: torch.device("cpu"))
+    monkeypatch.setattr(ops, "stream_of", lambda device: 0)
+    monkeypatch.setattr(ops, "call", lambda name, *args: calls.setdefault(name, args))
+    odd = lambda *shape: torch.zeros(1 + torch.Size(shape).numel())[1:].view(shape)
+    n, d = 24, 64
+    w, scale, keep = torch.zeros(d, 32), odd(d), None
+    x, g, stats = odd(n, d), odd(n, d), torch.zeros(n, 4)
+    assert all(t.data_ptr() % 16 for t in (x, g, scale))
+    kv = ops.gate_residual_rows(x, odd(n, 32), w, w, scale, scale, ME_GATE_SCALAR_SQRT, keep, True, True, True)[3]
+    ops.gate_rows_backward(g, x, kv[:, :d], kv[:, d:], scale, scale, ME_GATE_SCALAR_SQRT, keep, stats)
+    ops.gate_rows_backward_workspace_bytes.cache_clear()
+    forward, backward = calls["me_gate_rows"], calls["me_gate_rows_backward"]
+    assert all(p % 16 == 0 for p in (*(forward[i] for i in (0, 4, 5, 8, 9)), *(backward[i] for i in (0, 4, 5, 8, 9, 13))))
+    # rows that are no multiple of 16 bytes gain nothing from a copy
+    x, k = odd(n, 36), torch.zeros(n, 36)
+    calls.clear()
+    ops.gate_rows_backward(x, x, k, k, None, None, ME_GATE_SCALAR, keep, stats)
+    ops.gate_rows_backward_workspace_bytes.cache_clear()
+    assert calls["me_gate_rows_backward"][0] == x.data_ptr()
