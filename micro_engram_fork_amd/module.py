@@ -117,14 +117,14 @@ class _GateResidual(torch.autograd.Function):
         ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv)
         ctx.gate_mode = gate_mode
         ctx.mark_non_differentiable(alpha)
-        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient
+        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient (for out's: backward)
         return out, alpha
 
     @staticmethod
     def backward(ctx, grad_out, _grad_alpha):
-        if grad_out is None:
-            return (None,) * len(ctx.needs_input_grad)
         hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, kv = ctx.saved_tensors
+        if grad_out is None:
+            grad_out = torch.zeros_like(hidden)
         need = ctx.needs_input_grad
         wk, wv = w_key.detach(), w_value.detach()
         q = None if q_delta is None else q_delta.detach()
@@ -178,14 +178,14 @@ class _GateResidualRows(torch.autograd.Function):
         ctx.save_for_backward(hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, k, v)
         ctx.gate_mode = gate_mode
         ctx.mark_non_differentiable(alpha)
-        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient
+        ctx.set_materialize_grads(False)  # no zeros are filled in for alpha's gradient (for out's: backward)
         return out, alpha
 
     @staticmethod
     def backward(ctx, grad_out, _grad_alpha):
-        if grad_out is None:
-            return (None,) * len(ctx.needs_input_grad)
         hidden, mem, w_key, w_value, q_delta, k_delta, keep, stats, k, v = ctx.saved_tensors
+        if grad_out is None:
+            grad_out = torch.zeros_like(hidden)
         need = ctx.needs_input_grad
         wk, wv = w_key.detach(), w_value.detach()
         g_hidden, g_key, g_value, g_q, g_k = ops.gate_rows_backward(

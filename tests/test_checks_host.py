@@ -126,3 +126,23 @@ def test_unaligned_operands_with_gradients_are_copied_once(monkeypatch):
     ops.gate_rows_backward(x, x, k, k, None, None, ME_GATE_SCALAR, keep, stats)
     ops.gate_rows_backward_workspace_bytes.cache_clear()
     assert calls["me_gate_rows_backward"][0] == x.data_ptr()
+
+
+@pytest.mark.parametrize("d", [64, 36])
+def test_an_output_whose_consumer_gives_no_gradient_leaves_gradients(launches, d):
+    # what the engram's parameters get then is a gradient (of zeros), as from a gradient of zeros
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.sum()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+
+    eng = _engram(d)
+    out = eng.gate_residual(torch.zeros(12, d), torch.zeros(12, 32))
+    NoGradient.apply(out).backward()
+    assert "me_gate_rows_backward" in launches
+    for p in (eng.key.weight, eng.value.weight, eng.q_scale, eng.k_scale):
+        assert p.grad is not None and p.grad.shape == p.shape
