@@ -29,10 +29,12 @@
 // component i of every lane (the sum runs over the same k in a permuted order in both operands).
 // fp32, many tiles: the fp32 matrix rate (157 TFLOP/s) bounds those, so a slab is one k-step of 32 on the
 // bf16 matrix cores. Each value is split exactly into three bf16 parts as its fragment is read (11
-// vector instructions per pair), and six of the nine products of the parts are accumulated in fp32;
-// the other three are below 2^-26 of each term. 2-norm error against 64 bits, normal values, memory dim
-// 512 / 1024 / 1536: 3.4e-7 / 4.8e-7 / 6.0e-7 (fp32 MFMAs 4.1e-7 / 5.7e-7 / 7.0e-7); the parts of values under
-// 2^-110 end below the smallest bf16. The splitting and the MFMAs take turns on a SIMD (2048
+// vector instructions per pair and one that checks the parts), and six of the nine products of the parts are
+// accumulated in fp32; the other three are below 2^-26 of each term. 2-norm error against 64 bits, normal
+// values, memory dim 512 / 1024 / 1536: 3.4e-7 / 4.8e-7 / 6.0e-7 (fp32 MFMAs 4.1e-7 / 5.7e-7 / 7.0e-7). Blocks of
+// 16 x 16 outputs with values that have no such parts (not finite, or so tiny, under about 2^-110, that the last
+// part ends below the smallest bf16) are made again in fp32 MFMAs: slower, 2048 tokens with one tiny weight
+// 107 us where they take 68 without. The splitting and the MFMAs take turns on a SIMD (2048
 // tokens at 1024 x 1024: 61.6 us, 24 of them MFMAs at their full rate): one wave with the next
 // slab's splitting placed between its MFMAs, 16x16x32 or 32x32x16, took as long.
 #include "me_common.h"
@@ -118,7 +120,9 @@ struct Split {
     u32x4_v p[3];
 };
 
-__device__ __forceinline__ Split split_of(const u32x4_v &lo, const u32x4_v &hi) {
+// `rest` collects the bits of what is left for the third part: that part is exact where the low half of
+// its fp32 is zero, which values under about 2^-110 may miss (the smallest bf16 is 2^-133).
+__device__ __forceinline__ Split split_of(const u32x4_v &lo, const u32x4_v &hi, uint32_t &rest) {
     Split s;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -129,6 +133,7 @@ __device__ __forceinline__ Split split_of(const u32x4_v &lo, const u32x4_v &hi) 
             // one v_cvt_pk_bf16_f32 for the pair
             const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){x, y}, bf16x2));
             s.p[t][i] = w;
+            if (t == 2) rest |= __float_as_uint(x) | __float_as_uint(y);
             x -= __uint_as_float(w << 16);
             y -= __uint_as_float(w & 0xffff0000u);
         }
@@ -222,6 +227,7 @@ __global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
     };
 
     const int slabs = a.slabs;
+    uint32_t rest_a[BA] = {}, rest_b[BB] = {};  // split_of's, of this lane's row of each block
 #pragma unroll
     for (int sl = 0; sl < R - 1; ++sl)
         if (sl < slabs) issue(sl);
@@ -240,12 +246,12 @@ __global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
 #pragma unroll
             for (int i = 0; i < BA; ++i) {
                 const int row = wa * 16 * BA + 16 * i + fr;
-                fa[i] = split_of(frag(slot, row, 0), frag(slot, row, 1));
+                fa[i] = split_of(frag(slot, row, 0), frag(slot, row, 1), rest_a[i]);
             }
 #pragma unroll
             for (int j = 0; j < BB; ++j) {
                 const int row = TM + wb * 16 * BB + 16 * j + fr;
-                fb[j] = split_of(frag(slot, row, 0), frag(slot, row, 1));
+                fb[j] = split_of(frag(slot, row, 0), frag(slot, row, 1), rest_b[j]);
             }
             // of the nine products of the parts the three below 2^-26 of the first are left out; the small
             // ones come first, each over every block before the next: an MFMA waits for its accumulator
@@ -272,13 +278,14 @@ __global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
         }
     }
     if constexpr (SPLIT) {
-        // A value that is not finite has no such parts (its remainder is NaN; that of a value whose
-        // rounding overflows is infinite), so blocks whose sums are not finite are made again from the values themselves, in fp32 MFMAs.
+        // A value that is not finite has no such parts (its remainder is NaN; that of a value whose rounding
+        // overflows is infinite), and a tiny one not all of them: blocks whose sums are not finite and blocks
+        // with parts that are not exact are made again from the values themselves, in fp32 MFMAs.
 #pragma unroll
         for (int i = 0; i < BA; ++i)
 #pragma unroll
             for (int j = 0; j < BB; ++j) {
-                bool bad = false;
+                bool bad = ((rest_a[i] | rest_b[j]) & 0xffffu) != 0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) bad |= (__float_as_uint(acc[i][j][r]) & 0x7f800000u) == 0x7f800000u;
                 if (__any(bad)) {
@@ -289,10 +296,17 @@ __global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
                     const float *pt = reinterpret_cast<const float *>(a.mem) + (live_t ? tok : 0) * a.m;
                     const float *pc = reinterpret_cast<const float *>(vc < a.d_pad ? a.wk : a.wv) + (live_c ? jr : 0) * a.m;
                     floatx4 sum = floatx4{0.f, 0.f, 0.f, 0.f};
-                    for (int64_t k0 = 0; k0 < a.m; k0 += 4) {  // m % 4 == 0
-                        const float x = live_t ? *as_global(pt + k0 + fq) : 0.f;
-                        const float y = live_c ? *as_global(pc + k0 + fq) : 0.f;
-                        sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, sum, 0, 0, 0);
+                    for (int64_t k0 = 0; k0 < a.m; k0 += 32) {  // m % 4 == 0; eight steps' loads in flight
+                        float x[8], y[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            const bool in = k0 + 4 * u < a.m;
+                            x[u] = in && live_t ? *as_global(pt + k0 + 4 * u + fq) : 0.f;
+                            y[u] = in && live_c ? *as_global(pc + k0 + 4 * u + fq) : 0.f;
+                        }
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], y[u], sum, 0, 0, 0);
                     }
                     acc[i][j] = sum;
                 }

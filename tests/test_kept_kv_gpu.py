@@ -102,6 +102,28 @@ def test_kv_proj_fp32_values_of_any_size(n, d):
     assert bool(((kv - ref).abs() <= 2.0 ** -24 * ref.abs() + (m + 1) * 2.0 ** -24 * mag).all())
 
 
+# values under about 2^-110 have no three bf16 parts: fp32 MFMAs, split products on both their tiles; memory
+# rows of whole and partial k-steps, a tiny row, a tiny column and single tiny values among others
+@pytest.mark.parametrize("n,d,m", [(70, 64, 64), (700, 1032, 64), (700, 1032, 36), (1025, 2056, 64), (1025, 2056, 200)])
+@pytest.mark.parametrize("exponent", [-104, -112, -124, -140, -146])
+def test_kv_proj_fp32_tiny_values(n, d, m, exponent):
+    g = torch.Generator(device=DEV).manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    mem, wk, wv = r(n, m), r(d, m), r(d, m)
+    tiny = 2.0 ** exponent
+    mem[n - 1] = (r(m).double() * tiny).float()
+    mem[3, 5] = tiny * 1.2345678
+    wk[d - 1] = (r(m).double() * tiny).float()
+    wv[7] *= 2.0 ** 20
+    wv[9, m - 1] = tiny
+    kv = ops.kv_proj(mem, wk, wv).double()
+    w = torch.cat([wk, wv]).double().t().contiguous()
+    ref, mag = mem.double() @ w, mem.double().abs() @ w.abs()
+    # each of the m products and sums is rounded once in fp32, at 2^-149 where it is subnormal
+    bound = 2.0 ** -24 * ref.abs() + (m + 1) * 2.0 ** -24 * mag + (m + 1) * 2.0 ** -149
+    assert bool(((kv - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1025, 2056)])
 def test_kv_proj_fp32_infinities_and_nan(n, d):
     # where a value is infinite or NaN, so is what the products give, and nothing else changes
