@@ -464,18 +464,24 @@ int launch_few(const ProjArgs &a, hipStream_t s) {
     return check_launch("me_kv_proj (few tokens)");
 }
 
-// Every workgroup reads every token's row, so the kernel pays while those reads are few: it takes 64
-// tokens of at most kFewBytes in all (us, few / ring tiles of 32 x 32; model dim x memory dim, bf16:
-// 5376 x 1536, 8 tokens 7.9 / 9.2, 16: 9.2 / 9.2, 32: 13.6 / 9.2; 2048 x 1024, 32: 5.2 / 6.1, 48: 6.8 / 6.2)
-// and rows of at most 48 slabs (96 KB of LDS).
-constexpr int64_t kFewTokens = 64;
-constexpr int64_t kFewBytes = 22'000'000;
+// Every workgroup reads every token's row, so the kernel pays while those reads are few (us, few / ring tiles
+// of 32 x 32; model dim x memory dim, bf16: 5376 x 1536, 8 tokens 7.9 / 9.2, 16: 9.2 / 9.2, 32: 13.6 / 9.2;
+// 2048 x 1024, 32: 5.2 / 6.1; 8192 x 512, 20: 6.2 / 5.3) and its token blocks are at most two: from 33 tokens bf16
+// takes the ring tiles (48 tokens: 2560 x 640 8.1 / 5.7, 5320 x 136 5.4 / 4.4, 1024 x 1024 6.7 / 6.5), fp32, whose
+// ring tiles are bound by their MFMAs, from 65 (2048 x 1024, 48: 14.2 / 17.2). Past 50 MB the weights take as
+// long either way (8192 x 2048 in bf16, 1 token: 13.6 / 12.6). Rows have at most 48 slabs (96 KB of LDS).
+bool takes_few(const ProjArgs &a, int dtype) {
+    if (a.n > (dtype == ME_BF16 ? 32 : 64) || a.slabs > 48) return false;
+    if (2 * a.d_pad * a.row_bytes > 50'000'000) return false;
+    return 2 * a.d_pad / 16 * a.n * a.row_bytes <= (a.n <= 16 || dtype != ME_BF16 ? 22'000'000 : 17'000'000);
+}
 
 template <typename T>
 int few(const ProjArgs &a, hipStream_t s) {
     if (a.n <= 16) return launch_few<T, 1>(a, s);
-    if (a.n <= 32) return launch_few<T, 2>(a, s);
-    return launch_few<T, 4>(a, s);
+    if constexpr (sizeof(T) == 4)
+        if (a.n > 32) return launch_few<T, 4>(a, s);
+    return launch_few<T, 2>(a, s);
 }
 
 template <typename T, int BA, int BB, int R, bool SPLIT = false, int WA = 2>
@@ -530,7 +536,8 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // 128-byte slabs (19 tokens: 9.2 us; 10.4 with 32 x 96 and four slots; at 2048 x 1024, 128
     // tokens: 6.9, 8.9), 64 x 64 with four (192 tokens: 13.2; 15.6 with 64 x 96; at 3584 x 1536, 256
     // tokens: 12.7, 15.4), 64 x 96 with four (256 tokens: 16.0; 64 x 64 20.3, 128 x 96 17.6, with eight
-    // waves 14.8 by itself but 0.2 us more in a decode step). Tiles of one round, one to a CU, take eight
+    // waves 14.8 by itself but 0.2 us more in a decode step; also where they make one round, 128 tokens: 12.8,
+    // 64 x 64 13.9). Tiles of one round, one to a CU, take eight
     // waves, two per SIMD as two smaller workgroups are, with fewer bytes for the same outputs: 64 x 64 with
     // six slots (48 tokens: 9.8, 10.5 with four waves, the decode step 24.6 -> 23.7; at 2048 x 1024, 256
     // tokens: 7.8, 8.2), 256 x 96 (512 tokens: 24.4, 29.1 in 64 x 128; the decode step of 500 tokens 46.7 ->
@@ -544,18 +551,19 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // at 2048 x 1024, 1024 tokens: 24.8, 14.9; 2048: 25.7, 27.1; 8192: 76.7, 107; at 1024 x 512, 2048
     // tokens: 16.9, 10.6). Both were measured against 128 x 192 tiles (512 tokens 29.2 us, 1024: 51.5,
     // 1237: 73.2, 8192: 363), which stay for many tokens of a memory width the first cannot take.
-    // fp32: fp32 MFMAs on 32 x 64 tiles while all of them find a place (us, model dim and memory dim
-    // 1024: 100 tokens 16.3, 18.4 split; 200: 16.9, 26.4; 300: 23.9, 27.0), then split products on 64 x 64
-    // (1000 tokens: 38.5; 40.9 in fp32 on 32 x 128) and on 64 x 128 ones (2048 tokens 61.6; fp32 71.7;
-    // 4096: 119, 140; 777 tokens at 2000 x 512: 32.4, 41.9; 4096 at 2048 x 1536: 344, 409).
-    if (n <= kFewTokens && a.slabs <= 48 && 2 * a.d_pad / 16 * n * a.row_bytes <= kFewBytes)
-        return dtype == ME_BF16 ? few<uint16_t>(a, s) : few<float>(a, s);
+    // fp32: fp32 MFMAs on 32 x 64 and 32 x 128 tiles, split products on 64 x 64 and 64 x 128 ones, whichever the
+    // rule below takes least time for: with c tiles on the fullest CU (two at a time) they take about 11, 19, 17.5
+    // and 29 us per c at a memory dim of 1024, and as much less or more as that is shorter or longer (us in that
+    // order, model dim x memory dim: 1024 x 1024, 200 tokens 17.4, 24.7, 27.2, 38.7, 512: 26.2, 25.5, 28.4, 39.5,
+    // 1000: 46.7, 41.5, 39.8, 40.6, 2048: 89.9, 78.4, 75.4, 63.1, where 64 x 128 tiles of fp32 MFMAs took 76-82;
+    // 3584 x 1536, 257: 65.7, 58.9, 81.2, 82.9; 2560 x 640, 800: 58.4, 50.6, 57.8, 58.0).
+    if (takes_few(a, dtype)) return dtype == ME_BF16 ? few<uint16_t>(a, s) : few<float>(a, s);
     constexpr int64_t kCus = 256;
     auto tiles = [&](int tokens, int cols) { return ceil_div(n, tokens) * ceil_div(2 * a.d_pad, cols); };
     if (dtype == ME_BF16) {
         if (tiles(32, 32) <= 2 * kCus) return launch<uint16_t, 1, 1, 6>(a, s);
         if (tiles(64, 64) <= kCus) return launch<uint16_t, 1, 2, 6, false, 4>(a, s);
-        if (tiles(64, 64) <= 2 * kCus) return launch<uint16_t, 2, 2, 4>(a, s);
+        if (tiles(64, 64) <= 2 * kCus && tiles(64, 96) > kCus) return launch<uint16_t, 2, 2, 4>(a, s);
         if (tiles(64, 96) <= 2 * kCus) return launch<uint16_t, 2, 3, 4>(a, s);
         if (tiles(64, 128) > 2 * kCus) {  // three rounds and more of those below
             if (tiles(256, 96) <= kCus) return launch<uint16_t, 4, 3, 3, false, 4>(a, s);
@@ -571,7 +579,13 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
         }
         return launch<uint16_t, 2, 4, 3>(a, s);
     }
-    if (tiles(32, 64) <= 2 * kCus) return launch<float, 1, 2, 5>(a, s);
-    if (tiles(64, 64) <= 2 * kCus) return launch<float, 2, 2, 4, true>(a, s);
-    return launch<float, 2, 4, 3, true>(a, s);
+    // a tile alone on its CU takes longer than its share of two
+    auto per_cu = [&](int tokens, int cols) { return fmaxf(1.3f, static_cast<float>(ceil_div(tiles(tokens, cols), kCus))); };
+    const float t32x64 = 11.f * per_cu(32, 64) + 3.5f, t32x128 = 19.f * per_cu(32, 128) + 4.5f;
+    const float t64x64 = 17.5f * per_cu(64, 64) + 5.f, t64x128 = 29.f * per_cu(64, 128) + 3.f;
+    const float least = fminf(fminf(t32x64, t32x128), fminf(t64x64, t64x128));
+    if (t32x64 == least) return launch<float, 1, 2, 5>(a, s);
+    if (t64x64 == least) return launch<float, 2, 2, 4, true>(a, s);
+    if (t64x128 == least) return launch<float, 2, 4, 3, true>(a, s);
+    return launch<float, 1, 4, 4>(a, s);
 }

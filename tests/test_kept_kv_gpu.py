@@ -69,7 +69,7 @@ def test_kv_proj_tiles(n, d, m):
     _check_proj(n, d, m, torch.bfloat16)
 
 
-# the few-token kernel: every count of 16-token blocks and its edges, columns that end inside a
+# the few-token kernel (bf16 up to 32 tokens, fp32 up to 64): every count of 16-token blocks and its edges, columns that end inside a
 # 16-column block, memory rows of one part of a slab, of fewer slabs than waves, of partial slabs,
 # of each slab count per wave (2, 4, 6, 8, 12) and past its widest (3200)
 @pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 32, 33, 64])
@@ -79,15 +79,16 @@ def test_kv_proj_few_tokens(n, d, m, dtype):
     _check_proj(n, d, m, dtype)
 
 
-# fp32 past the few-token kernel: fp32 MFMAs on tiles of 32 x 64, split products on 64 x 64 and 64 x 128, by
-# the tiles they make; memory rows of whole and partial slabs, columns and tokens that end inside a tile
+# fp32 past the few-token kernel: fp32 MFMAs on tiles of 32 x 64 and 32 x 128 (the last two), split products on
+# 64 x 64 (1000 tokens) and 64 x 128, by the tiles they make; memory rows of whole and partial slabs, columns and
+# tokens that end inside a tile
 @pytest.mark.parametrize("n,d,m", [(65, 264, 1536), (300, 1024, 200), (700, 1032, 96), (1000, 1024, 36), (1025, 1024, 64),
-                                   (2049, 520, 4), (1025, 2056, 200)])
+                                   (2049, 520, 4), (1025, 2056, 200), (257, 3576, 36), (800, 2560, 100)])
 def test_kv_proj_fp32_tiles(n, d, m):
     _check_proj(n, d, m, torch.float32)
 
 
-@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1025, 2056)])
+@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1000, 1024), (1025, 2056)])
 def test_kv_proj_fp32_values_of_any_size(n, d):
     # rows and columns scaled by 2^-40 .. 2^40: the split is exact at every exponent, so the bound of
     # _check_proj holds relative to each element's own magnitudes
@@ -104,7 +105,7 @@ def test_kv_proj_fp32_values_of_any_size(n, d):
 
 # values under about 2^-110 have no three bf16 parts: fp32 MFMAs, split products on both their tiles; memory
 # rows of whole and partial k-steps, a tiny row, a tiny column and single tiny values among others
-@pytest.mark.parametrize("n,d,m", [(70, 64, 64), (700, 1032, 64), (700, 1032, 36), (1025, 2056, 64), (1025, 2056, 200)])
+@pytest.mark.parametrize("n,d,m", [(70, 64, 64), (1000, 1024, 64), (1000, 1024, 36), (1025, 2056, 64), (1025, 2056, 200)])
 @pytest.mark.parametrize("exponent", [-104, -112, -124, -140, -146])
 def test_kv_proj_fp32_tiny_values(n, d, m, exponent):
     g = torch.Generator(device=DEV).manual_seed(5)
@@ -124,7 +125,7 @@ def test_kv_proj_fp32_tiny_values(n, d, m, exponent):
     assert bool(((kv - ref).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1025, 2056)])
+@pytest.mark.parametrize("n,d", [(70, 64), (700, 1032), (1000, 1024), (1025, 2056)])
 def test_kv_proj_fp32_infinities_and_nan(n, d):
     # where a value is infinite or NaN, so is what the products give, and nothing else changes
     m = 64
