@@ -549,8 +549,8 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     // slab, 256 tiles of the second 1.2 us and 0.33 us per slab, but never under 1.6 such (512
     // tokens: 33.4 and 30.5 us; 768: 33.7, 36.7; 1237: 39.0, 61.6; 2048: 69.9, 101; 8192: 233, 398;
     // at 2048 x 1024, 1024 tokens: 24.8, 14.9; 2048: 25.7, 27.1; 8192: 76.7, 107; at 1024 x 512, 2048
-    // tokens: 16.9, 10.6). Both were measured against 128 x 192 tiles (512 tokens 29.2 us, 1024: 51.5,
-    // 1237: 73.2, 8192: 363), which stay for many tokens of a memory width the first cannot take.
+    // tokens: 16.9, 10.6). 64 x 128 also where the memory width rules the first out (5320 x 136, 4096 tokens:
+    // 43.2; 55.5 on 128 x 192 tiles, which were slower than one of the others for every shape measured).
     // fp32: fp32 MFMAs on 32 x 64 and 32 x 128 tiles, split products on 64 x 64 and 64 x 128 ones, whichever the
     // rule below takes least time for: with c tiles on the fullest CU (two at a time) they take about 11, 19, 17.5
     // and 29 us per c at a memory dim of 1024, and as much less or more as that is shorter or longer (us in that
@@ -574,8 +574,6 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
             const float large = static_cast<float>(ceil_div(ceil_div(n, 256) * 2 * ceil_div(model_dim, 224), kCus));
             if (large * (7.f + 1.25f * a.slabs) <= 2.f + fmaxf(small, 1.6f) * (1.2f + 0.33f * a.slabs))
                 return kv_proj_224(mem, n, mem_dim, w_key, w_value, model_dim, kv, s);
-        } else if (tiles(128, 192) > 2 * kCus) {
-            return launch<uint16_t, 4, 6, 4>(a, s);
         }
         return launch<uint16_t, 2, 4, 3>(a, s);
     }

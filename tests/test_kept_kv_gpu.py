@@ -69,6 +69,12 @@ def test_kv_proj_tiles(n, d, m):
     _check_proj(n, d, m, torch.bfloat16)
 
 
+# many tokens of memory rows that are no whole slabs (64 x 128 tiles past every one-round tile), with a row end
+# inside a slab and columns that end inside a tile
+def test_kv_proj_many_tokens_of_partial_slabs():
+    _check_proj(1153, 5320, 136, torch.bfloat16)
+
+
 # the few-token kernel (bf16 up to 32 tokens, fp32 up to 64): every count of 16-token blocks and its edges, columns that end inside a
 # 16-column block, memory rows of one part of a slab, of fewer slabs than waves, of partial slabs,
 # of each slab count per wave (2, 4, 6, 8, 12) and past its widest (3200)
