@@ -18,7 +18,7 @@
 //
 // Any width: rows whose model dim, row stride or addresses do not allow 16-byte accesses take a
 // kernel that walks one column per lane and step (scalar loads and stores; 8 columns for rows over
-// 8064 columns and for hidden states of another dtype than the projections), so an engram of any
+// 8064 columns), so an engram of any
 // model dim and memory width runs (its projections then come from a library GEMM, the nn.Linear
 // of module.py:245, 254, since the MFMA kernels need whole 16-byte rows).
 //
@@ -479,7 +479,9 @@ __global__ __launch_bounds__(kThreads) void gate_rows_grad_kernel(const RowArgs 
 // registers and the workgroup writes one row of partials (the token at a time kernel above re-reads
 // hidden, g and K after the reduction, and a kernel of its own reads hidden and K again for the
 // scale gradients). 8192 tokens x 5376 in bf16, 616 MB: 246 us with that kernel, 132 with this one
-// (4.7 TB/s; a copy of 1 GiB reaches 5.1); 2048 x 1024 in fp32: 85 and 18. The stores are
+// (4.7 TB/s; a copy of 1 GiB reaches 5.1); 2048 x 1024 in fp32: 85 and 18. Hidden states of another dtype than the
+// projections gain as much (forward and backward with the projections and products, fp32 hidden and a bf16
+// engram, 5320 x 136, 8192 tokens: 780 us with that kernel, 633 with this one). The stores are
 // non-temporal (2048 x 5376: 36.5 us through the caches, 32 past them).
 template <typename H, typename T, int kRowThreads, int kSteps, bool kScaled>
 __global__ __launch_bounds__(kRowThreads) void gate_rows_grad_block_kernel(const RowArgs a, int per) {
@@ -727,45 +729,52 @@ size_t rows_grad_workspace(int64_t n, int64_t d) {
     return coef + static_cast<size_t>(parts) * static_cast<size_t>(d) * 4;
 }
 
-// Whether the one-pass kernels take these rows: hidden and the projections of one dtype (other
-// combinations stay on the kernels that take a column count per lane), at most kMaxGroups groups.
-bool one_pass(const RowArgs &a, int hidden_dtype, int dtype) {
-    return hidden_dtype == dtype && a.d <= kMaxGroups * kGroupCols;
-}
+// Whether the one-pass kernels take these rows: at most kMaxGroups groups.
+bool one_pass(const RowArgs &a) { return a.d <= kMaxGroups * kGroupCols; }
 
-template <typename T, int kRowThreads, int kSteps>
+template <typename H, typename T, int kRowThreads, int kSteps>
 void launch_row(const RowArgs &a, int per, unsigned groups, hipStream_t s) {
     if (a.grad_out == nullptr)
-        hipLaunchKernelGGL((gate_row_kernel<T, T, kRowThreads, kSteps>), dim3(groups), dim3(kRowThreads), 0, s, a);
+        hipLaunchKernelGGL((gate_row_kernel<H, T, kRowThreads, kSteps>), dim3(groups), dim3(kRowThreads), 0, s, a);
     else if (a.sqrt_mode)
-        hipLaunchKernelGGL((gate_rows_grad_block_kernel<T, T, kRowThreads, kSteps, true>), dim3(groups),
+        hipLaunchKernelGGL((gate_rows_grad_block_kernel<H, T, kRowThreads, kSteps, true>), dim3(groups),
                            dim3(kRowThreads), 0, s, a, per);
     else
-        hipLaunchKernelGGL((gate_rows_grad_block_kernel<T, T, kRowThreads, kSteps, false>), dim3(groups),
+        hipLaunchKernelGGL((gate_rows_grad_block_kernel<H, T, kRowThreads, kSteps, false>), dim3(groups),
                            dim3(kRowThreads), 0, s, a, per);
 }
 
 // The fewest steps with at most 24 groups (384 threads) each, and as few waves as hold them: every
 // load of a token in flight and few idle lanes (8192 tokens in bf16: 5376 columns, 48 groups, 63 us on
 // 2 x 384 threads and 77 on 1024; 1024 columns, 17 us on 256 threads and 46 on 1024).
-template <typename T>
+template <typename H, typename T>
 void launch_rows(const RowArgs &a, int per, unsigned groups, hipStream_t s) {
     const int g = static_cast<int>(ceil_div(a.d, 2 * kGroupCols)) * 2;
     const int steps = (g + 23) / 24;
     const int waves = static_cast<int>(ceil_div(ceil_div(g, steps), 4));
     if (steps == 1) {
-        if (waves <= 2) launch_row<T, 128, 1>(a, per, groups, s);
-        else if (waves == 3) launch_row<T, 192, 1>(a, per, groups, s);
-        else if (waves == 4) launch_row<T, 256, 1>(a, per, groups, s);
-        else if (waves == 5) launch_row<T, 320, 1>(a, per, groups, s);
-        else launch_row<T, 384, 1>(a, per, groups, s);
+        if (waves <= 2) launch_row<H, T, 128, 1>(a, per, groups, s);
+        else if (waves == 3) launch_row<H, T, 192, 1>(a, per, groups, s);
+        else if (waves == 4) launch_row<H, T, 256, 1>(a, per, groups, s);
+        else if (waves == 5) launch_row<H, T, 320, 1>(a, per, groups, s);
+        else launch_row<H, T, 384, 1>(a, per, groups, s);
     } else if (steps == 2) {
-        if (waves <= 4) launch_row<T, 256, 2>(a, per, groups, s);
-        else if (waves == 5) launch_row<T, 320, 2>(a, per, groups, s);
-        else launch_row<T, 384, 2>(a, per, groups, s);
+        if (waves <= 4) launch_row<H, T, 256, 2>(a, per, groups, s);
+        else if (waves == 5) launch_row<H, T, 320, 2>(a, per, groups, s);
+        else launch_row<H, T, 384, 2>(a, per, groups, s);
     } else {
-        if (waves <= 5) launch_row<T, 320, 3>(a, per, groups, s);
-        else launch_row<T, 384, 3>(a, per, groups, s);
+        if (waves <= 5) launch_row<H, T, 320, 3>(a, per, groups, s);
+        else launch_row<H, T, 384, 3>(a, per, groups, s);
+    }
+}
+
+void launch_rows(const RowArgs &a, int hidden_dtype, int dtype, int per, unsigned groups, hipStream_t s) {
+    if (hidden_dtype == ME_BF16) {
+        if (dtype == ME_BF16) launch_rows<uint16_t, uint16_t>(a, per, groups, s);
+        else launch_rows<uint16_t, float>(a, per, groups, s);
+    } else {
+        if (dtype == ME_BF16) launch_rows<float, uint16_t>(a, per, groups, s);
+        else launch_rows<float, float>(a, per, groups, s);
     }
 }
 
@@ -790,12 +799,10 @@ extern "C" int me_gate_rows(const void *hidden, int hidden_dtype, int64_t n, int
     hipStream_t s = as_stream(stream);
     if (!wide_rows(a, {hidden, k_proj, v_proj, out, a.q_delta, a.k_delta}))
         ME_ROWS_DISPATCH(gate_rows_kernel, 1, grid, s, a);
-    else if (!one_pass(a, hidden_dtype, dtype))
+    else if (!one_pass(a))
         ME_ROWS_DISPATCH(gate_rows_kernel, 8, grid, s, a);
-    else if (dtype == ME_BF16)
-        launch_rows<uint16_t>(a, 1, static_cast<unsigned>(n), s);
     else
-        launch_rows<float>(a, 1, static_cast<unsigned>(n), s);
+        launch_rows(a, hidden_dtype, dtype, 1, static_cast<unsigned>(n), s);
     return check_launch("me_gate_rows");
 }
 
@@ -845,11 +852,10 @@ extern "C" int me_gate_rows_backward(const void *hidden, int hidden_dtype, int64
     const dim3 grid(static_cast<unsigned>(n));
     const bool wide = wide_rows(a, {hidden, k_proj, v_proj, grad_out, grad_hidden, grad_key, grad_value, a.q_delta,
                                     a.k_delta});
-    if (wide && aligned16(row_stats) && one_pass(a, hidden_dtype, dtype)) {
+    if (wide && aligned16(row_stats) && one_pass(a)) {
         const int per = static_cast<int>(ceil_div(n, grad_groups(n, model_dim)));
         const unsigned groups = static_cast<unsigned>(ceil_div(n, per));
-        if (dtype == ME_BF16) launch_rows<uint16_t>(a, per, groups, s);
-        else launch_rows<float>(a, per, groups, s);
+        launch_rows(a, hidden_dtype, dtype, per, groups, s);
         const int bs = check_launch("me_gate_rows_backward (rows)");
         if (bs != ME_OK || !a.sqrt_mode) return bs;
         hipLaunchKernelGGL(gate_rows_scale_sum_kernel, dim3(static_cast<unsigned>(ceil_div(model_dim, 64))),

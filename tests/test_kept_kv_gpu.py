@@ -189,3 +189,28 @@ def test_kept_and_recomputed_gradients_agree(dtype, hidden_dtype):
     tol = 5e-2 if torch.bfloat16 in (dtype, hidden_dtype) else 5e-3
     for a, b in zip(*grads):
         assert a.dtype == b.dtype and (a.double() - b.double()).norm() <= tol * b.double().norm() + 1e-12
+
+
+# hidden states and projections of two dtypes whose values fit bf16: the sums are those of one dtype, and results
+# differ by their own rounding only. Model dims of each step count of the row kernels and their edges; 1100 tokens
+# are more than one per workgroup of the backward
+@pytest.mark.parametrize("n,d,mode", [
+    (37, 8, ME_GATE_SCALAR_SQRT), (37, 112, ME_GATE_SCALAR), (1100, 232, ME_GATE_SCALAR_SQRT), (37, 2688, ME_GATE_SCALAR_SQRT),
+    (37, 2696, ME_GATE_SCALAR), (37, 5376, ME_GATE_SCALAR_SQRT), (37, 5384, ME_GATE_SCALAR_SQRT), (37, 8064, ME_GATE_SCALAR_SQRT)])
+@pytest.mark.parametrize("hidden_dtype,dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+def test_rows_of_two_dtypes(n, d, mode, hidden_dtype, dtype):
+    x, mem, wk, wv, dq, dk, keep, g = _case(n, d, 64, mode, torch.bfloat16)
+    k, v = mem @ wk.t(), mem @ wv.t()
+    want = ops.gate_rows(x, k, v, dq, dk, mode, keep, True, True)
+    grads = ops.gate_rows_backward(g, x, k, v, dq, dk, mode, keep, want[2])
+    xm, gm, km, vm = x.to(hidden_dtype), g.to(hidden_dtype), k.to(dtype), v.to(dtype)
+    got = ops.gate_rows(xm, km, vm, dq, dk, mode, keep, True, True)
+    back = ops.gate_rows_backward(gm, xm, km, vm, dq, dk, mode, keep, want[2])
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])  # gates and sums
+    assert all(torch.equal(a.bfloat16(), b) for a, b in zip(back[1:3], grads[1:3]))  # of K and V: one rounding
+    assert all((a - b).norm() <= 1e-5 * b.norm() + 1e-12 for a, b in zip(back[3:], grads[3:]))
+    if hidden_dtype == torch.bfloat16:
+        assert torch.equal(got[0], want[0]) and torch.equal(back[0], grads[0])
+    else:  # bf16 rounds the term and the sum: at most 2^-8 of each
+        for a, b, base in ((got[0], want[0], xm), (back[0], grads[0], gm)):
+            assert bool(((a - b.float()).abs() <= 2.0 ** -8 * ((a - base).abs() + a.abs()) * 1.01 + 1e-30).all())
