@@ -557,11 +557,19 @@ class MicroEngram(nn.Module):
     # forward and backward of 2048 fp32 tokens at 1024 0.92 against 1.43.
     keep_kv_bytes = 1 << 30
 
+    # Columns of the widest rows that one pass of the row kernels takes (gate_rows.hip). Wider bf16 rows are
+    # read twice, which the fused kernels' recomputing beats where their tiles fill the part: those keep K and V
+    # up to few_tokens_max tokens only (forward and backward in us, recomputed / kept: model dim 9216, memory dim
+    # 256, 300 tokens 363 / 204, 16000: 1546 / 1749; 8072 x 512, 2048 tokens 378 / 389, 3000: 432 / 524).
+    keep_kv_columns = 8064
+
     def _keeps_kv(self, hidden, mem):
         """Whether a forward with gradients writes K and V out and keeps them (few_tokens_max = 0 keeps
         every call on the fused kernels, with or without gradients)."""
         few = self.few_tokens_max if mem.dtype == torch.bfloat16 else self.few_tokens_max_fp32
         n = hidden.numel() // hidden.shape[-1]
+        if hidden.shape[-1] > self.keep_kv_columns and n > self.few_tokens_max and mem.dtype == torch.bfloat16:
+            return False
         return n < 1 << 24 and few > 0 and 2 * hidden.numel() * mem.element_size() <= self.keep_kv_bytes
 
     def inject(self, hidden, idx, keep=None):

@@ -146,3 +146,13 @@ def test_an_output_whose_consumer_gives_no_gradient_leaves_gradients(launches, d
     assert "me_gate_rows_backward" in launches
     for p in (eng.key.weight, eng.value.weight, eng.q_scale, eng.k_scale):
         assert p.grad is not None and p.grad.shape == p.shape
+
+
+@pytest.mark.parametrize("d,n,dtype,kept", [
+    (8064, 1030, torch.bfloat16, True), (8072, 1024, torch.bfloat16, True), (8072, 1025, torch.bfloat16, False),
+    (8072, 1025, torch.float32, True)])
+def test_rows_past_one_pass_of_the_row_kernels_keep_k_and_v_for_few_tokens(launches, d, n, dtype, kept):
+    eng = _engram(d, dtype)
+    eng.gate_residual(torch.empty(n, d, dtype=dtype), torch.empty(n, 32, dtype=dtype)).sum().backward()
+    assert (launches[:2] == ["me_kv_proj", "me_gate_rows"]) == kept
+    assert ("me_gate_residual" in launches) == (not kept) and ("me_gate_backward" in launches) == (not kept)
