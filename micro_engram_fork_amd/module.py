@@ -559,8 +559,8 @@ class MicroEngram(nn.Module):
 
     # Columns of the widest rows that one pass of the row kernels takes (gate_rows.hip). Wider bf16 rows are
     # read twice, which the fused kernels' recomputing beats where their tiles fill the part: those keep K and V
-    # up to few_tokens_max tokens only (forward and backward in us, recomputed / kept: model dim 9216, memory dim
-    # 256, 300 tokens 363 / 204, 16000: 1546 / 1749; 8072 x 512, 2048 tokens 378 / 389, 3000: 432 / 524).
+    # up to 512 tokens only (forward and backward in us, recomputed / kept: model dim 9216, memory dim 256,
+    # 16000 tokens 1546 / 1749; 8072 x 512, 300 tokens 203 / 199, 700: 234 / 245, 1024: 236 / 262, 3000: 432 / 524).
     keep_kv_columns = 8064
 
     def _keeps_kv(self, hidden, mem):
@@ -568,7 +568,7 @@ class MicroEngram(nn.Module):
         every call on the fused kernels, with or without gradients)."""
         few = self.few_tokens_max if mem.dtype == torch.bfloat16 else self.few_tokens_max_fp32
         n = hidden.numel() // hidden.shape[-1]
-        if hidden.shape[-1] > self.keep_kv_columns and n > self.few_tokens_max and mem.dtype == torch.bfloat16:
+        if hidden.shape[-1] > self.keep_kv_columns and n > 512 and mem.dtype == torch.bfloat16:
             return False
         return n < 1 << 24 and few > 0 and 2 * hidden.numel() * mem.element_size() <= self.keep_kv_bytes
 
