@@ -594,12 +594,12 @@ class MicroEngram(nn.Module):
         and the row reads as one launch: the fused kernel without gradients, the same one leaving its
         row ids for the backward with them. Where lookup, hash_ids or inject has been replaced, or a
         server's lookup reads the rows, forward goes through those."""
-        if self._lookup_replaced() or (self.row_lookup_fn is not None and self.row_shards is not None):
+        if (self._lookup_replaced() or self._replaced("hash_ids") or self._replaced("inject")
+                or (self.row_lookup_fn is not None and self.row_shards is not None)):
             return self.inject(hidden, self.hash_ids(input_ids.to(hidden.device), position_ids))
         if not self._needs_grad(hidden):
             return self._gate(hidden, self.hashed_memory(input_ids, position_ids, hidden.device), None)
-        if (torch.compiler.is_compiling() or input_ids.numel() == 0 or self._replaced("hash_ids")
-                or self._replaced("inject")):
+        if torch.compiler.is_compiling() or input_ids.numel() == 0:
             return self.inject(hidden, self.hash_ids(input_ids.to(hidden.device), position_ids))
         device = hidden.device
         ids = input_ids.to(device)

@@ -156,3 +156,24 @@ def test_rows_past_one_pass_of_the_row_kernels_keep_k_and_v_for_few_tokens(launc
     eng.gate_residual(torch.empty(n, d, dtype=dtype), torch.empty(n, 32, dtype=dtype)).sum().backward()
     assert (launches[:2] == ["me_kv_proj", "me_gate_rows"]) == kept
     assert ("me_gate_residual" in launches) == (not kept) and ("me_gate_backward" in launches) == (not kept)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("name", ["hash_ids", "inject", "lookup"])
+def test_forward_goes_through_replaced_methods(launches, name, grad):
+    # set on the instance or overridden by a subclass, with and without gradients
+    seen = []
+
+    def replacement(self, *args, **kwargs):
+        seen.append(name)
+        return getattr(MicroEngram, name)(self, *args, **kwargs)
+
+    kw = dict(table_size=97, engram_dim=8, num_heads=2, orders=(2, 3), vocab_size=500, gate="scalar_sqrt")
+    subclass = type("Sub", (MicroEngram,), {name: replacement})(64, **kw)
+    instance = _engram(64)
+    setattr(instance, name, lambda *a, **k: replacement(instance, *a, **k))
+    hidden, ids = torch.zeros(1, 6, 64), torch.zeros(1, 6, dtype=torch.long)
+    for eng in (subclass, instance):
+        with torch.set_grad_enabled(grad):
+            eng(hidden, ids)
+    assert seen == [name, name]
