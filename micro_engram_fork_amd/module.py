@@ -484,8 +484,7 @@ class MicroEngram(nn.Module):
         return self._replaced("lookup")
 
     def _replaced(self, name):
-        cls = type(self)
-        return name in self.__dict__ or (cls is not MicroEngram and getattr(cls, name) is not getattr(MicroEngram, name))
+        return name in self.__dict__ or getattr(type(self), name) is not getattr(MicroEngram, name)
 
     # -------------------------------------------------------------------------------- inject
     def _needs_grad(self, hidden):
