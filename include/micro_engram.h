@@ -196,7 +196,11 @@ int me_gate_residual_noalloc(const void *hidden, int hidden_dtype, int64_t n, in
  *   mem       [n, mem_dim] of dtype (ME_BF16 / ME_F32); w_key, w_value [model_dim, mem_dim]
  *   kv        [n, 2 model_dim] of dtype
  * model_dim a multiple of 8, mem_dim * element size a multiple of 16 bytes, every tensor
- * 16-byte aligned, mem and each weight under 2 GiB. Together with me_gate_rows it is faster than
+ * 16-byte aligned, mem and each weight under 2 GiB, fewer than 2^24 tokens. The order of a sum depends on
+ * n (up to 32 tokens of bf16 and 64 of fp32 add four parts of mem_dim, more take one run), so the same row
+ * in batches of different sizes can differ in its last bit. fp32 batches of many tiles multiply exact bf16
+ * parts of each value, without the products below 2^-26 of a term; values that have no such parts (not
+ * finite, or under about 2^-110) are multiplied in fp32. Together with me_gate_rows it is faster than
  * me_gate_residual for small batches (a serving decode step) and where that kernel's 256-token
  * tiles leave CUs idle, and it keeps K and V for a backward; large batches without gradients
  * belong to me_gate_residual.
@@ -209,7 +213,7 @@ int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const void *w_key, c
  * computed elsewhere (me_kv_proj's output). Replaces the rest of
  * MicroEngram.inject after the two nn.Linear calls (micro_engram/module.py:240-261), with the
  * same arithmetic as me_gate_residual (for bf16 rows of up to 8064 columns its sums also run in
- * the order of that function's 224-column tiles, so both give the same bits):
+ * the order of that function's 224-column tiles, so both give the same bits from the same K and V):
  *
  *   h = rms_norm(hidden) [* (1 + q_scale_delta)], k = rms_norm(K) [* (1 + k_scale_delta)]
  *   s = sum(h k) / sqrt(model_dim); ME_GATE_SCALAR_SQRT: s = sign(s) sqrt(max(|s|, 1e-6))

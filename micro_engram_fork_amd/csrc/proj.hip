@@ -352,7 +352,7 @@ __global__ __launch_bounds__(128 * WA) void proj_kernel(const ProjArgs a) {
 }
 
 // ---- a few tokens: every weight byte in flight at once ---------------------------------------------
-// Up to kFewTokens tokens the GEMM is one read of the weights (33 MB at the Gemma-scale shape) and next to
+// For a few tokens (takes_few) the GEMM is one read of the weights (33 MB at the Gemma-scale shape) and next to
 // no arithmetic, so what counts is how soon all of it is in flight: a tile's ring (above) keeps three
 // slabs of its rows in flight and walks 24, a chain of eight memory latencies. Here a workgroup takes
 // 16 columns whole: its four waves split the slabs, each wave asks for all of its rows' lines at
@@ -513,7 +513,7 @@ extern "C" int me_kv_proj(const void *mem, int64_t n, int64_t mem_dim, const voi
     ME_CHECK_ARG((mem_dim * es) % 16 == 0, "mem_dim * element size must be a multiple of 16 bytes");
     ME_CHECK_ARG(n * mem_dim * es < (int64_t{1} << 31) && model_dim * mem_dim * es < (int64_t{1} << 31),
                  "mem and each weight must be under 2 GiB");
-    ME_CHECK_ARG(n < (int64_t{1} << 24), "too many tokens for the few-token projection");
+    ME_CHECK_ARG(n < (int64_t{1} << 24), "too many tokens: at most 2^24 - 1");
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     ME_CHECK_ARG(al16(mem) && al16(w_key) && al16(w_value) && al16(kv), "tensors must be 16-byte aligned");
     ProjArgs a{};

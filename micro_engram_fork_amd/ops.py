@@ -421,8 +421,8 @@ def _(hidden, mem, w_key, w_value, q_scale_delta, k_scale_delta, gate_mode, keep
 @_custom_op("kv_proj")
 def kv_proj(mem: torch.Tensor, w_key: torch.Tensor, w_value: torch.Tensor) -> torch.Tensor:
     """[K | V] [N, 2d] in mem's dtype: the key and value nn.Linear outputs of
-    MicroEngram.inject (module.py:245, 254) for few tokens, in one hand-written MFMA kernel
-    (me_kv_proj). mem [N, M]; w_key, w_value [d, M] (nn.Linear layout)."""
+    MicroEngram.inject (module.py:245, 254), in one hand-written MFMA kernel (me_kv_proj).
+    mem [N, M]; w_key, w_value [d, M] (nn.Linear layout)."""
     dev = require_gpu(mem, w_key, w_value)
     if mem.dim() != 2 or w_key.dim() != 2 or w_key.shape != w_value.shape or w_key.shape[1] != mem.shape[1]:
         raise ValueError(f"[micro_engram] kv_proj: mem {tuple(mem.shape)} and weights {tuple(w_key.shape)}/"
@@ -457,7 +457,9 @@ def prefers_rows(n, model_dim, mem_dim):
     kernel (gate_rows) than in the fused kernel, for shapes both take (whole 128-byte slabs of the
     memory rows, at least three).
 
-    Both run 256 x 224 tiles, one per CU, so their time goes by whole rounds of 256 tiles: the fused
+    The estimate knows the projection's 256 x 224 and 64 x 128 tiles, not its one-round tiles between them, which
+    take less than either, so it keeps some calls on the fused kernel that the other would serve as well; of some
+    200 calls of 21 shapes that it moved none was slower for it. Both run 256 x 224 tiles, one per CU, so their time goes by whole rounds of 256 tiles: the fused
     kernel makes one set of rounds per pass (key, value), the projection one set for both together,
     then K and V cross the memory once each way. A round of the fused kernel's two passes takes
     about 25 us and 2.2 us per slab, one of the projection 7 and 1.25 (or less on small tiles),

@@ -126,7 +126,7 @@ class _KeyPlan:
     def bounds(self):
         """[count, table bounds] as host ints."""
         self.make()
-        if self.host is None:
+        if self.host is None:  # read before, by a backward that failed afterwards
             return self.info.tolist()
         self.ready.synchronize()
         buf, self.host = self.host, None
