@@ -459,7 +459,9 @@ def prefers_rows(n, model_dim, mem_dim):
 
     The estimate knows the projection's 256 x 224 and 64 x 128 tiles, not its one-round tiles between them, which
     take less than either, so it keeps some calls on the fused kernel that the other would serve as well; of some
-    200 calls of 21 shapes that it moved none was slower for it. Both run 256 x 224 tiles, one per CU, so their time goes by whole rounds of 256 tiles: the fused
+    200 calls of 21 shapes that it moved none was slower for it.
+
+    Both run 256 x 224 tiles, one per CU, so their time goes by whole rounds of 256 tiles: the fused
     kernel makes one set of rounds per pass (key, value), the projection one set for both together,
     then K and V cross the memory once each way. A round of the fused kernel's two passes takes
     about 25 us and 2.2 us per slab, one of the projection 7 and 1.25 (or less on small tiles),

@@ -75,8 +75,8 @@ def test_kv_proj_many_tokens_of_partial_slabs():
     _check_proj(1153, 5320, 136, torch.bfloat16)
 
 
-# the few-token kernel (bf16 up to 32 tokens, fp32 up to 64): every count of 16-token blocks and its edges, columns that end inside a
-# 16-column block, memory rows of one part of a slab, of fewer slabs than waves, of partial slabs,
+# the few-token kernel (bf16 up to 32 tokens, fp32 up to 64): every count of 16-token blocks and its edges, columns
+# that end inside a 16-column block, memory rows of one part of a slab, of fewer slabs than waves, of partial slabs,
 # of each slab count per wave (2, 4, 6, 8, 12) and past its widest (3200)
 @pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("d,m", [(8, 16), (24, 192), (1032, 200), (40, 896), (264, 1536), (16, 2048), (8, 3072), (8, 3200)])
